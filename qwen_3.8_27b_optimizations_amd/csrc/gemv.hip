@@ -1135,31 +1135,24 @@ hipError_t launch_gemv_group(int count, const uint8_t* const* W, float* const* Y
     for (int i = 0; i < count; ++i) mats[i] = {W[i], Y[i], N[i], layout_mk ? N[i] : 1};
     const int64_t ldy_n = layout_mk ? 1 : M;
     static const int kind = tuning_knob("IQ4XS_GEMV_KIND", 2, 0, 2);
-    // matrix-core matrices first, one launch per wave count (the same
-    // routing and kernel as single calls)
+    // the matrix-core matrices share launches (the same routing and kernel as single calls)
     TileMat rest[GEMV_GROUP_MAX];
-    int n_rest = 0;
-    bool done[GEMV_GROUP_MAX] = {};
+    const uint8_t* gW[GEMV_GROUP_MAX];
+    float* gY[GEMV_GROUP_MAX];
+    int64_t gN[GEMV_GROUP_MAX], gL[GEMV_GROUP_MAX];
+    int n = 0, n_rest = 0;
     for (int i = 0; i < count; ++i) {
-        if (done[i]) continue;
         if (!use_gemv_mfma(N[i], M)) {
             rest[n_rest++] = mats[i];
             continue;
         }
-        const uint8_t* gW[GEMV_GROUP_MAX];
-        float* gY[GEMV_GROUP_MAX];
-        int64_t gN[GEMV_GROUP_MAX], gL[GEMV_GROUP_MAX];
-        int n = 0;
-        const int waves = gemv_mfma_waves(N[i]);
-        for (int j = i; j < count; ++j) {
-            if (done[j] || !use_gemv_mfma(N[j], M) || gemv_mfma_waves(N[j]) != waves) continue;
-            gW[n] = W[j];
-            gY[n] = Y[j];
-            gN[n] = N[j];
-            gL[n] = mats[j].ldy_m;
-            ++n;
-            done[j] = true;
-        }
+        gW[n] = W[i];
+        gY[n] = Y[i];
+        gN[n] = N[i];
+        gL[n] = mats[i].ldy_m;
+        ++n;
+    }
+    if (n > 0) {
         hipError_t err = launch_gemv_mfma_group(n, gW, gY, gN, gL, aqs, ads, K, M, ldy_n, nullptr, stream);
         if (err == hipErrorNotSupported) {  // shapes past its offsets take the single-call route
             err = hipSuccess;

@@ -1,5 +1,5 @@
-// gemv_mfma.hip -- small-batch IQ4_XS x Q8_1 GEMV (2 <= M <= 8 columns) on
-// the gfx950 int8 matrix cores.
+// gemv_mfma.hip -- small-batch IQ4_XS x Q8_1 multiply (2 <= M <= GM_MAX_COLS
+// columns) on the gfx950 int8 matrix cores.
 //
 // Semantics: those of the GEMV / GEMM (real_stock_dp4a_comparator.hip:
 // 68-166, 374-443): per 32-weight sub-block the exact int32 dot sumi of the
@@ -7,33 +7,40 @@
 // column's fp16 d.
 //
 // Why a second GEMV.  The dot4 GEMV spends VALU work per weight byte and per
-// column, so from 4 columns on it is VALU-bound (bs = 8 ran at 1.35 TB/s).
-// Here one v_mfma_i32_32x32x32_i8 takes 32 weight rows x 32 k of one
-// sub-block against all columns at once (the A operand is the activations,
-// one token per MFMA row; rows past M hold any token and only produce C rows
-// that are never stored), so the VALU cost per weight byte no longer grows
-// with M: decoding the codes into the B operand, then per useful output a
-// convert, a scale product and a fused add.
+// column, so from 4 columns on it is VALU-bound.  Here one
+// v_mfma_i32_32x32x32_i8 takes 32 weight rows x 32 k of one sub-block against
+// up to 32 columns (the A operand is the activations, one token per MFMA row;
+// rows past M hold any token and only produce C rows that are never stored),
+// so the VALU cost is the decode of the codes into the B operand, the same for
+// any M, and per output a subtract, a scale product and a fused add.
 //
-// Mapping.  A workgroup of GM_WAVES (8 or 16) waves owns up to 32 weight rows
-// (one MFMA block; rows past its own are masked); its waves take
-// the super-blocks kb = wave, wave + GM_WAVES, ... (at any moment they stream
-// GM_WAVES consecutive super-blocks of the same rows), each wave keeping one
-// super-block of loads in flight while it computes the previous one.  Its
-// loads are coalesced (each of the 4 weight loads covers the qs of 8 whole
-// rows, the 2 activation loads a token's 256 codes per 8 lanes) and staged in
-// LDS rows of the wave's own, from which the MFMA operands are read.  The
-// MFMA sums over k, so any order of k that A and B share gives the same
-// int32: lane l (half h = l >> 5) supplies weight row l & 31 with both
-// nibbles of qs bytes 8h .. 8h+7 of the sub-block (sub-block weights
-// 8h .. 8h+7 and 16+8h .. 16+8h+7), decoded in registers, and the A lanes the
-// activation codes of the same 16 weights.  The C element e of lane l is
-// token 8*(e>>2) + 4h + (e&3) of that row.  The token scales of a
-// super-block ride in the activation ring (one ds word per lane) and are
-// staged with its codes, so no workgroup-wide prologue or barrier precedes
-// the stream (staging every column scale up front measured 3-12 % slower).
-// The GM_WAVES partial sums of every output are added in LDS in wave order
-// (deterministic).
+// Mapping.  A workgroup owns up to 32 weight rows (one MFMA block) of one
+// matrix and 8 G tokens, and splits K over its waves: wave w takes the
+// super-blocks kb = w, w + waves, ... (at any moment the waves stream adjacent
+// super-blocks of the same rows), with no barrier before the final sum.  The
+// partial sums are added in wave order and the wave count follows the
+// matrix's own shape (gm_waves), so a row's bits depend neither on the rows
+// per workgroup nor on what shares the launch.
+//   * Loads are coalesced (each of the 4 weight loads of a block covers the qs
+//     of 8 whole rows, the activation loads a token's 256 codes per 8 lanes)
+//     and staged in LDS rows of the wave's own, from which the MFMA operands
+//     are read.  Staging frees the load registers, so the next block's loads
+//     are issued before the current block is computed, without a second set
+//     (112 VGPRs at G = 2; the two-set form this replaces measured 20.7 us
+//     against 18.6 us on 17408 -> 5120 at M = 8).
+//   * The MFMA sums over k, so any order of k that A and B share gives the same
+//     int32: lane l (half h = l >> 5) supplies weight row l & 31 with both
+//     nibbles of qs bytes 8h .. 8h+7 of the sub-block (weights 8h .. 8h+7 and
+//     16+8h .. 16+8h+7), and the A lanes the activation codes of the same 16
+//     weights, which the staging puts side by side (one 16-byte read).
+//   * The C element e of lane l is token 8*(e>>2) + 4h + (e&3) of its row.
+//   * The int32 sum comes back as a float without a convert (which issues at
+//     half the rate of an add): the accumulator starts at the bits of
+//     1/(2 pi) = 0x3E22F983, an inline constant in the middle of the binade
+//     [1/8, 1/4), so that sumi (|sumi| < 2^20) counts units of 2^-26 there and
+//     one exact subtraction leaves sumi * 2^-26; the weight scale carries 2^26.
+#include <algorithm>
+
 #include "iq4xs_device.h"
 #include "iq4xs_internal.h"
 
@@ -41,52 +48,46 @@ namespace iq4xs {
 
 constexpr int GM_LDS_MAX = 160 * 1024;
 
-constexpr int GM_AROW = 272;  // LDS row of one token's 256 codes, padded (bank spread)
-constexpr int GM_WROW = 144;  // LDS row of one weight row's 128 qs bytes, padded
+constexpr int GM_AROW = 272;  // LDS row of one token's 256 codes, padded (conflict-free 16-byte reads)
+constexpr int GM_WROW = 136;  // LDS row of one weight row's 128 qs bytes, padded (conflict-free 8-byte reads)
 // per-wave staging bytes: weight rows, token rows, then the super-block's
-// column scales [8 sub-blocks][8 tokens]
-constexpr int GM_WAVE_LDS = 32 * GM_WROW + 8 * GM_AROW + 8 * 8 * 4;
-// Register ring of weight super-blocks per wave (one in flight while one is
-// computed); the activations, read by every workgroup and so L2-resident,
-// have a ring of their own, also one super-block ahead.  Depths 3 and 4
-// measured slower (more VGPRs, no better overlap).
-constexpr int GM_RING = 2;
+// column scales [8 sub-blocks][8G tokens]; the final sum reuses them
+constexpr int gm_wave_lds(int G) { return 32 * GM_WROW + G * (8 * GM_AROW + 8 * 8 * 4); }
 
-struct GmW {      // weights of one super-block (from HBM: the deep ring)
-    v2u h;       // d, scales_h, scales_l of this lane's row's super-block
-    v4i q[4];    // qs chunk (lane % 8) of rows lane/8 + 8i: 8 whole rows per load instruction
-};
-struct GmA {      // activations of one super-block (L2-resident: one ahead)
-    v4i a[2];    // 32 of the super-block's activation codes: token lane/8, bytes 32*(lane%8) ..
-    uint32_t ds; // Q8_1 ds word of token lane/8, sub-block lane%8
-};
+constexpr int GM_ZERO_BITS = 0x3E22F983;  // the accumulator's zero (1/(2 pi) as a float)
+
+// Most waves of a workgroup (gm_waves).
+constexpr int gm_max_waves(int G) { return G <= 2 ? 16 : 8; }
+// Waves per SIMD that the registers are held to (96, 114, 146 and 152 VGPRs).
+constexpr int gm_waves_per_simd(int G, bool debug) { return G == 1 ? 5 : (G == 2 ? 4 : (debug ? 2 : 3)); }
 
 // The matrices of one launch (same K and activations): workgroups
-// [tile_end[i-1], tile_end[i]) run matrix i, rows[i] rows each.  Entries past
-// the group's count repeat its last matrix with tile_end = the grid size, so
-// no workgroup selects them.
+// [tile_end[i-1], tile_end[i]) run matrix i.  Entries past the group's count
+// repeat its last matrix with tile_end = the grid size, so no workgroup
+// selects them.
 struct GmGroup {
     const uint8_t* W[GEMV_GROUP_MAX];
     float* Y[GEMV_GROUP_MAX];
     int64_t ldy_m[GEMV_GROUP_MAX];
     int N[GEMV_GROUP_MAX];
-    int rows[GEMV_GROUP_MAX];
     int tile_end[GEMV_GROUP_MAX];
 };
 
-template <int GM_WAVES, bool kDebug>
-__global__ __launch_bounds__(64 * GM_WAVES) void gemv_mfma_kernel(const GmGroup grp,
-                                                                  const int8_t* __restrict__ aqs,
-                                                                  const uint32_t* __restrict__ ads, int K, int M,
-                                                                  int64_t ldy_n, int32_t* __restrict__ dbg) {
-    constexpr int G = 1;  // M <= 8: tokens 4h + e of element e < 4
-    extern __shared__ __attribute__((aligned(16))) float gm_lds[];
+template <int G, bool kDebug>
+__global__ __launch_bounds__(64 * gm_max_waves(G)) __attribute__((amdgpu_waves_per_eu(gm_waves_per_simd(G, kDebug))))
+void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const uint32_t* __restrict__ ads, int K,
+                      int M, int rows, int toks, int64_t ldy_n, int32_t* __restrict__ dbg) {
+    // sub-blocks unrolled together: all 8, fewer where the registers of their
+    // reads in flight would cost a wave per SIMD (M = 32, gate + up: 2 together
+    // 56.6 us, 1 at a time 50.6)
+    constexpr int UNR = kDebug || G == 4 ? 1 : (G == 3 ? 2 : 8);
+    extern __shared__ __attribute__((aligned(16))) uint8_t gm_lds[];
     // this workgroup's matrix: scalar selects on the by-value descriptor (a
     // dynamic index into it would go through scratch)
     const uint8_t* __restrict__ W = grp.W[0];
     float* __restrict__ Y = grp.Y[0];
     int64_t ldy_m = grp.ldy_m[0];
-    int N = grp.N[0], rows = grp.rows[0], tile0 = 0;
+    int N = grp.N[0], tile0 = 0;
 #pragma unroll
     for (int i = 1; i < GEMV_GROUP_MAX; ++i) {
         if ((int)blockIdx.x >= grp.tile_end[i - 1]) {
@@ -94,190 +95,220 @@ __global__ __launch_bounds__(64 * GM_WAVES) void gemv_mfma_kernel(const GmGroup 
             Y = grp.Y[i];
             ldy_m = grp.ldy_m[i];
             N = grp.N[i];
-            rows = grp.rows[i];
             tile0 = grp.tile_end[i - 1];
         }
     }
     const int bpr = K / QK_K, nb = K / QK8_1;
-    float* red = gm_lds;                        // [GM_WAVES][4G][64] partial sums
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, col = lane & 31;
-    uint8_t* swave = reinterpret_cast<uint8_t*>(red + GM_WAVES * 4 * G * 64) + (tid >> 6) * GM_WAVE_LDS;
-    uint8_t* sw = swave;                                          // [32][144] qs of the 32 rows
-    int8_t* sact = reinterpret_cast<int8_t*>(swave + 32 * GM_WROW);  // [8][272] activations
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = (int)blockDim.x >> 6;
+    uint8_t* sw = gm_lds + wave * gm_wave_lds(G);                   // [32][136] qs of a block's rows
+    uint8_t* sact = sw + 32 * GM_WROW;                              // [8G][272] activations
+    float* sdx = reinterpret_cast<float*>(sact + 8 * G * GM_AROW);  // [8][8G] column scales (0 past M)
     const int r0 = ((int)blockIdx.x - tile0) * rows;
-    const int nrow = min(rows, N - r0);  // this workgroup's rows (1..32; MFMA rows past them are masked)
-    // Global loads are 32-bit lane offsets from workgroup-uniform bases (a
-    // 32-row block spans 32 * K/256 * 136 bytes), which keeps the load ring
-    // in VGPRs.  MFMA rows past nrow are clamped to its last row (a repeat
-    // of bytes already loaded, so no extra HBM traffic): computed, never stored.
+    const int nrow = min(rows, N - r0);  // this workgroup's rows (1 .. 32)
+    const int t0 = (int)blockIdx.y * toks;
+    const int mt = min(toks, M - t0);  // this workgroup's tokens (1 .. 8G)
+    // Global loads are 32-bit lane offsets from workgroup-uniform bases.  MFMA
+    // rows past nrow are clamped to its last row (a repeat of bytes already
+    // loaded, so no extra HBM traffic): computed, never stored.
     const uint32_t row_bytes = (uint32_t)bpr * BLOCK_BYTES;
     const uint8_t* wbase = W + (size_t)r0 * row_bytes;
-    const uint32_t off_h = (uint32_t)min(col, nrow - 1) * row_bytes;     // this lane's row (header)
-    uint32_t off_q[4];                                                    // rows lane/8 + 8i, qs chunk lane%8
+    const int8_t* abase = aqs + (size_t)t0 * K;
+    const uint32_t* dbase = ads + (size_t)t0 * nb;
+
+    // an offset kept scalar: the loads then take a scalar base and a 32-bit
+    // lane offset, instead of a 64-bit address per lane and load
+    auto uniform = [](int off) {
+        asm volatile("" : "+s"(off));
+        return (uint32_t)off;
+    };
+    v2u wh;        // d, scales_h, scales_l of row col
+    v4i wq[4];     // qs chunk lane % 8 of rows lane/8 + 8i
+    v4i xa[G][2];  // sub-block lane % 8 of token 8g + lane/8
+    uint32_t xd[G];
+    auto load_w = [&](int kb) {
+        const uint8_t* wk = wbase + uniform(kb * BLOCK_BYTES);
+        wh = *reinterpret_cast<const v2u*>(wk + (uint32_t)min(col, nrow - 1) * row_bytes);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        off_q[i] = (uint32_t)min((lane >> 3) + 8 * i, nrow - 1) * row_bytes + 8 + 16 * (lane & 7);
+        for (int i = 0; i < 4; ++i)
+            wq[i] = *reinterpret_cast<const v4i_a8*>(
+                wk + ((uint32_t)min(8 * i + (lane >> 3), nrow - 1) * row_bytes + 8 + 16 * (lane & 7)));
+    };
+    auto load_x = [&](int kb) {
+        const int8_t* ak = abase + uniform(kb * QK_K);
+        const uint32_t* dk = dbase + uniform(kb * 8);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const uint32_t t = (uint32_t)min(8 * g + (lane >> 3), mt - 1);
+            const uint32_t off = t * (uint32_t)K + 32 * (lane & 7);
+            xa[g][0] = *reinterpret_cast<const v4i*>(ak + off);
+            xa[g][1] = *reinterpret_cast<const v4i*>(ak + off + 16);
+            xd[g] = dk[t * (uint32_t)nb + (lane & 7)];
+        }
+    };
+    // LDS operations of one wave complete in order: the reads below by other
+    // lanes of the wave see these writes, and the previous block's reads were
+    // issued before them
+    uint8_t* xwrite = sact + (lane >> 3) * GM_AROW + 32 * (lane & 7);
+    const uint8_t* xread = sact + min(col, 8 * G - 1) * GM_AROW + 16 * h;
     uint8_t* wwrite = sw + (lane >> 3) * GM_WROW + 16 * (lane & 7);
     const uint8_t* wread = sw + col * GM_WROW + 8 * h;
-    // this lane's share of a super-block's activations, and its MFMA A row in LDS
-    const uint32_t off_a = (uint32_t)min(lane >> 3, M - 1) * (uint32_t)K + 32 * (lane & 7);
-    int8_t* awrite = sact + (lane >> 3) * GM_AROW + 32 * (lane & 7);
-    const int8_t* aread = sact + min(col, M - 1) * GM_AROW + 8 * h;
-    // the current super-block's column scales, [sub-block][token] (0 past M),
-    // and this lane's ds word in every super-block: token lane/8, sub-block lane%8
-    float* sdx = reinterpret_cast<float*>(sact + 8 * GM_AROW);
-    const uint32_t off_d = (uint32_t)min(lane >> 3, M - 1) * (uint32_t)nb + (lane & 7);
-
-    const int my_n = wave < bpr ? (bpr - wave + GM_WAVES - 1) / GM_WAVES : 0;
-    auto load_w = [&](GmW& p, int kb) {
-        const uint8_t* wk = wbase + (size_t)kb * BLOCK_BYTES;   // uniform
-        p.h = *reinterpret_cast<const v2u*>(wk + off_h);
+    auto stage_x = [&]() {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) p.q[i] = *reinterpret_cast<const v4i_a8*>(wk + off_q[i]);
+        for (int g = 0; g < G; ++g) {
+            // elements 0-7, 16-23 and 8-15, 24-31: the A operand of each lane half
+            *reinterpret_cast<v4i*>(xwrite + 8 * g * GM_AROW) = v4i{xa[g][0].x, xa[g][0].y, xa[g][1].x, xa[g][1].y};
+            *reinterpret_cast<v4i*>(xwrite + 8 * g * GM_AROW + 16) =
+                v4i{xa[g][0].z, xa[g][0].w, xa[g][1].z, xa[g][1].w};
+            const int t = 8 * g + (lane >> 3);
+            sdx[(lane & 7) * 8 * G + t] = t < mt ? half_bits_to_float(xd[g] & 0xFFFFu) : 0.0f;
+        }
     };
-    auto load_a = [&](GmA& p, int kb) {
-        const int8_t* ak = aqs + (size_t)kb * QK_K;               // uniform
-        p.a[0] = *reinterpret_cast<const v4i*>(ak + off_a);
-        p.a[1] = *reinterpret_cast<const v4i*>(ak + off_a + 16);
-        p.ds = ads[(size_t)kb * 8 + off_d];
+    auto stage_w = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            *reinterpret_cast<v2u*>(wwrite + 8 * i * GM_WROW) = v2u{(uint32_t)wq[i].x, (uint32_t)wq[i].y};
+            *reinterpret_cast<v2u*>(wwrite + 8 * i * GM_WROW + 8) = v2u{(uint32_t)wq[i].z, (uint32_t)wq[i].w};
+        }
     };
 
     float acc[4 * G];
 #pragma unroll
     for (int e = 0; e < 4 * G; ++e) acc[e] = 0.0f;
-    auto compute = [&](const GmW& p, const GmA& pa, int kb) {
-        // the wave's own LDS rows: written here, read below by other lanes of
-        // the same wave (LDS operations of one wave complete in order; the
-        // previous super-block's reads were issued before these writes)
-        *reinterpret_cast<v4i*>(awrite) = pa.a[0];
-        *reinterpret_cast<v4i*>(awrite + 16) = pa.a[1];
-        sdx[(lane & 7) * 8 + (lane >> 3)] = (lane >> 3) < M ? half_bits_to_float(pa.ds & 0xFFFFu) : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<v4i*>(wwrite + 8 * i * GM_WROW) = p.q[i];
-        const float dw = half_bits_to_float(p.h.x & 0xFFFFu);
-#pragma unroll
+    auto compute = [&](const v2u hd, int kb) {
+        const float dw = half_bits_to_float(hd.x & 0xFFFFu) * 67108864.0f;  // 2^26
+#pragma unroll UNR
         for (int s = 0; s < 8; ++s) {
             uint32_t lo0, hi0, lo1, hi1;
             const v2u q = *reinterpret_cast<const v2u*>(wread + 16 * s);
             decode_codes_x(q.x, lo0, hi0);
             decode_codes_x(q.y, lo1, hi1);
-            const v4i b = v4i{(int)lo0, (int)lo1, (int)hi0, (int)hi1};
-            const v2u a0 = *reinterpret_cast<const v2u*>(aread + 32 * s);
-            const v2u a1 = *reinterpret_cast<const v2u*>(aread + 32 * s + 16);
-            const v4i a = v4i{(int)a0.x, (int)a0.y, (int)a1.x, (int)a1.y};
-            const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, v16i{}, 0, 0, 0);
-            const int ls = subblock_ls(p.h.x, p.h.y, s) - 32;
+            const v4i bw = v4i{(int)lo0, (int)lo1, (int)hi0, (int)hi1};
+            const v4i ax = *reinterpret_cast<const v4i*>(xread + 32 * s);
+            v16i z;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) z[e] = GM_ZERO_BITS;
+            const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(ax, bw, z, 0, 0, 0);
+            const int ls = subblock_ls(hd.x, hd.y, s) - 32;
             const float sa = dw * (float)ls;
-            const float* bxp = sdx + s * 8 + 4 * h;
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const v4f bx = *reinterpret_cast<const v4f*>(bxp + 8 * g);
+                const v4f bx = *reinterpret_cast<const v4f*>(sdx + s * 8 * G + 8 * g + 4 * h);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int e = 4 * g + j;
-                    acc[e] = __builtin_fmaf((float)c[e], sa * bx[j], acc[e]);
+                    const float f = __builtin_bit_cast(float, (int)c[e]) - __builtin_bit_cast(float, GM_ZERO_BITS);
+                    acc[e] = __builtin_fmaf(f, sa * bx[j], acc[e]);
                     if (kDebug) {
                         const int t = 8 * g + 4 * h + j;
-                        if (t < M && col < nrow) dbg[((size_t)t * N + r0 + col) * nb + kb * 8 + s] = c[e] * ls;
+                        if (t < mt && col < nrow)
+                            dbg[((size_t)(t0 + t) * N + r0 + col) * nb + kb * 8 + s] =
+                                ((int)c[e] - GM_ZERO_BITS) * ls;
                     }
                 }
             }
         }
     };
-    // ring of GM_RING super-blocks with constant indices (unrolled by its
-    // depth); every load is unconditional (past this wave's last super-block
-    // it repeats that one)
-    // the loop is unrolled by 2 * GM_RING so that both rings have constant
-    // indices (registers, not scratch)
-    constexpr int UNR = 2 * GM_RING;
-    GmW wb[GM_RING];
-    GmA ab[2];
-    if (my_n > 0) {
-#pragma unroll
-        for (int d = 0; d < GM_RING - 1; ++d) load_w(wb[d], wave + GM_WAVES * min(d, my_n - 1));
-        load_a(ab[0], wave);
-    }
-    for (int i0 = 0; i0 < my_n; i0 += UNR) {
-#pragma unroll
-        for (int d = 0; d < UNR; ++d) {
-            const int i = i0 + d;
-            if (i0 + d >= my_n && d > 0) break;  // uniform: no loads past the last round's end
-            load_w(wb[(d + GM_RING - 1) % GM_RING], wave + GM_WAVES * min(i + GM_RING - 1, my_n - 1));
-            load_a(ab[(d + 1) % 2], wave + GM_WAVES * min(i + 1, my_n - 1));
-            if (i < my_n) compute(wb[d % GM_RING], ab[d % 2], wave + GM_WAVES * i);
+    // every load is unconditional (past this wave's last super-block it repeats that one)
+    if (wave < bpr) {
+        load_x(wave);
+        load_w(wave);
+        for (int kb = wave; kb < bpr; kb += waves) {
+            const int kn = kb + waves < bpr ? kb + waves : kb;
+            const v2u hd = wh;
+            stage_x();
+            load_x(kn);
+            stage_w();
+            load_w(kn);
+            compute(hd, kb);
         }
     }
+    // the waves' partial sums, added in wave order
+    __syncthreads();  // the staging is free
+    float* red = reinterpret_cast<float*>(gm_lds);  // [waves][4G][64]
+    constexpr int PER = 4 * G * 64;
+    static_assert(PER * 4 <= gm_wave_lds(G), "the final sum fits the staging");
 #pragma unroll
-    for (int e = 0; e < 4 * G; ++e) red[(wave * 4 * G + e) * 64 + lane] = acc[e];
+    for (int e = 0; e < 4 * G; ++e) red[wave * PER + e * 64 + lane] = acc[e];
     __syncthreads();
-    if (wave == 0 && col < nrow) {
-#pragma unroll
-        for (int e = 0; e < 4 * G; ++e) {
-            float v = red[e * 64 + lane];
-#pragma unroll
-            for (int w = 1; w < GM_WAVES; ++w) v += red[(w * 4 * G + e) * 64 + lane];
-            const int t = 8 * (e >> 2) + 4 * h + (e & 3);
-            if (t < M) Y[t * ldy_m + (int64_t)(r0 + col) * ldy_n] = v;
+    for (int e = wave; e < 4 * G; e += waves) {  // uniform per wave
+        float v = red[e * 64 + lane];
+        for (int w = 1; w < waves; ++w) v += red[w * PER + e * 64 + lane];
+        const int t = 8 * (e >> 2) + 4 * h + (e & 3);
+        if (t < mt && col < nrow) Y[(int64_t)(t0 + t) * ldy_m + (int64_t)(r0 + col) * ldy_n] = v;
+    }
+}
+
+// Tokens: blocks of at most 32, as even as possible.
+static int64_t gm_token_blocks(int64_t M) { return (M + 31) / 32; }
+static int64_t gm_tokens(int64_t M) { return (M + gm_token_blocks(M) - 1) / gm_token_blocks(M); }
+
+// Waves per workgroup of an N-row matrix.  They fix a row's fp32 summation
+// order, so they follow the matrix's own shape and M, never the launch.
+//   * From 384 row blocks on (gate/up, N = 17408) the blocks alone nearly fill
+//     the chip: 8 waves each, 4 past 16 tokens, where the registers allow 12
+//     waves per CU.  Below, K is split further so that every CU has loads in
+//     flight: 12 waves, 16 from K = 8192 on (as fast, with shorter sums), or 8
+//     past 16 tokens.  Measured (us per launch, 4 / 8 /
+//     12 waves): gate + up M = 8 30.6 / 30.3 / 33.4, M = 32 54.3 / 63.6 / 68.9;
+//     17408 -> 5120 M = 8 32.5 / 21.0 / 18.7 (16 waves: 19.1), M = 32 48.7 / 32.0 / 33.5; q/k/v
+//     M = 16 16.8 / 16.4 / 17.4.
+static int gm_waves(int64_t N, int64_t K, int G) {
+    const int64_t bpr = K / QK_K;
+    const int w = (N + 31) / 32 >= 384 ? (G <= 2 ? 8 : 4) : (G <= 2 && bpr < 32 ? 12 : gm_max_waves(G));
+    return (int)std::max<int64_t>(4, std::min<int64_t>(w, bpr));
+}
+
+template <int G>
+static hipError_t launch_gm(const GmGroup& grp, dim3 grid, int waves, const int8_t* aqs, const uint32_t* ads,
+                            int64_t K, int64_t M, int64_t rows, int64_t toks, int64_t ldy_n, int32_t* dbg,
+                            hipStream_t stream) {
+    const size_t lds = (size_t)waves * gm_wave_lds(G);
+    static_assert(gm_max_waves(G) * gm_wave_lds(G) <= GM_LDS_MAX, "the staging fits a CU");
+    auto launch = [&](auto kernel) -> hipError_t {
+        if (lds > 64 * 1024) {  // beyond the default dynamic-LDS limit of a launch
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS_MAX);
+            if (e != hipSuccess) return e;
         }
-    }
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), lds, stream, grp, aqs, ads, (int)K, (int)M, (int)rows,
+                           (int)toks, ldy_n, dbg);
+        return hipGetLastError();
+    };
+    return dbg ? launch(&gemv_mfma_kernel<G, true>) : launch(&gemv_mfma_kernel<G, false>);
 }
 
-// Workgroups and rows per workgroup of one matrix.  The wave count fixes each
-// row's fp32 summation order; the rows per workgroup only balance the grid (a
-// row's arithmetic does not depend on them).
-struct GmPlan {
-    int waves, rows;
-};
-
-static GmPlan gm_plan(int64_t N) {
-    // Parallelism comes from splitting K over the waves of a row block: with
-    // fewer 32-row blocks than two per CU, 16 waves each (measured: q, o and
-    // down 5-15 % faster), otherwise 8 (gate/up: 16 would leave fewer
-    // workgroups resident per CU).  With 16 waves the rows per workgroup (at
-    // most 32, the MFMA's) are chosen so that every CU gets the same number
-    // of workgroups: N = 5120 takes 20 rows on 256 CUs instead of 160 blocks
-    // of 32 that leave 96 CUs idle (bs = 8: down 21.3 -> 18.4-19.5 us, o
-    // unchanged).  Each workgroup decodes all 32 MFMA rows whatever it keeps,
-    // so the 8-wave shapes stay at 32 rows (gate with 17-row workgroups, 4
-    // per CU instead of 2.125: 18.9 -> 21.5 us).
-    //
-    // The wave count is chosen from the shape alone, against MI355X's 256
-    // CUs, so a device or partition with another CU count gives the same
-    // bits; the rows per workgroup use the device's own CU count.
-    constexpr int64_t kWaveChoiceCus = 256;
-    const int64_t cus = device_cu_count();
-    if ((N + 31) / 32 < 2 * kWaveChoiceCus) {
-        const int64_t k = (N + 32 * cus - 1) / (32 * cus);
-        // at least 8 rows: narrow matrices (k/v, N = 1024, at 8 columns)
-        // measured 6.60 us with 8-row workgroups against 6.99 with 4
-        const int64_t rows = (N + cus * k - 1) / (cus * k);
-        return {16, (int)(rows < 8 ? 8 : rows)};
+// The matrices of one wave count in one launch.
+static hipError_t launch_gm_waves(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
+                                  const int64_t* ldy_m, const int8_t* aqs, const uint32_t* ads, int64_t K, int64_t M,
+                                  int64_t ldy_n, int32_t* dbg, int waves, hipStream_t stream) {
+    const int64_t tblocks = gm_token_blocks(M), toks = gm_tokens(M), cus = device_cu_count();
+    // Rows per workgroup: 32, fewer where that leaves CUs without one (N =
+    // 5120: 20 rows on 256 CUs against 160 blocks of 32); at least 8, since
+    // each workgroup decodes all 32 MFMA rows whatever it keeps (N = 1024, M =
+    // 8: 6.6 us with 8 rows against 7.0 with 4).
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) total += N[i];
+    const int64_t rows = std::max<int64_t>(8, std::min<int64_t>(32, (total * tblocks + cus - 1) / cus));
+    GmGroup grp{};
+    int64_t wgs = 0;
+    for (int i = 0; i < GEMV_GROUP_MAX; ++i) {
+        const int j = i < count ? i : count - 1;
+        if (i < count) wgs += (N[j] + rows - 1) / rows;
+        if (wgs > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
+        grp.W[i] = W[j];
+        grp.Y[i] = Y[j];
+        grp.ldy_m[i] = ldy_m[j];
+        grp.N[i] = (int)N[j];
+        grp.tile_end[i] = (int)wgs;
     }
-    return {8, 32};
-}
-
-template <int WAVES>
-static hipError_t launch_gm(const GmGroup& grp, int64_t wgs, const int8_t* aqs, const uint32_t* ads, int64_t K,
-                            int64_t M, int64_t ldy_n, int32_t* dbg, hipStream_t stream) {
-    const size_t lds = (size_t)WAVES * 4 * 64 * sizeof(float) + (size_t)WAVES * GM_WAVE_LDS;
-    if (lds > GM_LDS_MAX) return hipErrorNotSupported;
-    if (lds > 64 * 1024) {  // beyond the default dynamic-LDS limit of a launch
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_mfma_kernel<WAVES, false>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS_MAX);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemv_mfma_kernel<WAVES, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, GM_LDS_MAX);
-        if (e != hipSuccess) return e;
+    const dim3 grid((unsigned)wgs, (unsigned)tblocks);
+    switch ((toks + 7) / 8) {
+        case 1: return launch_gm<1>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
+        case 2: return launch_gm<2>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
+        case 3: return launch_gm<3>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
+        default: return launch_gm<4>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
     }
-    const dim3 grid((unsigned)wgs), block(64 * WAVES);
-    if (dbg)
-        hipLaunchKernelGGL((gemv_mfma_kernel<WAVES, true>), grid, block, lds, stream, grp, aqs, ads, (int)K, (int)M,
-                           ldy_n, dbg);
-    else
-        hipLaunchKernelGGL((gemv_mfma_kernel<WAVES, false>), grid, block, lds, stream, grp, aqs, ads, (int)K, (int)M,
-                           ldy_n, dbg);
-    return hipGetLastError();
 }
 
 hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
@@ -285,33 +316,36 @@ hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* con
                                   int64_t M, int64_t ldy_n, int32_t* dbg, hipStream_t stream) {
     clear_launch_error();
     if (count < 1 || count > GEMV_GROUP_MAX || (dbg && count != 1)) return hipErrorInvalidValue;
-    if (M < 1 || M > 8 || K % QK_K || K >= (1 << 24)) return hipErrorNotSupported;
-    // the kernel's 32-bit load offsets span one 32-row block and 8 token rows
-    if ((int64_t)32 * (K / QK_K) * BLOCK_BYTES >= ((int64_t)1 << 31) || (int64_t)8 * K >= ((int64_t)1 << 31))
+    if (M < 1 || M > GM_MAX_COLS || K % QK_K || K >= (1 << 24)) return hipErrorNotSupported;
+    // the kernel's 32-bit load offsets span 32 rows and 32 tokens
+    if ((int64_t)32 * (K / QK_K) * BLOCK_BYTES >= ((int64_t)1 << 31) || (int64_t)32 * K >= ((int64_t)1 << 31))
         return hipErrorNotSupported;
-    GmGroup grp{};
-    int64_t wgs = 0;
-    int waves = 0;
-    for (int i = 0; i < GEMV_GROUP_MAX; ++i) {
-        const int j = i < count ? i : count - 1;
-        if (N[j] < 1 || N[j] >= (1 << 30)) return hipErrorNotSupported;
-        const GmPlan plan = gm_plan(N[j]);
-        if (i == 0) waves = plan.waves;
-        if (plan.waves != waves) return hipErrorNotSupported;  // one wave count per launch
-        if (i < count) wgs += (N[j] + plan.rows - 1) / plan.rows;
-        if (wgs > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
-        grp.W[i] = W[j];
-        grp.Y[i] = Y[j];
-        grp.ldy_m[i] = ldy_m[j];
-        grp.N[i] = (int)N[j];
-        grp.rows[i] = plan.rows;
-        grp.tile_end[i] = (int)wgs;
+    for (int i = 0; i < count; ++i)
+        if (N[i] < 1 || N[i] >= (1 << 30)) return hipErrorNotSupported;
+    // one launch per wave count
+    const int G = (int)((gm_tokens(M) + 7) / 8);
+    bool done[GEMV_GROUP_MAX] = {};
+    for (int i = 0; i < count; ++i) {
+        if (done[i]) continue;
+        const int waves = gm_waves(N[i], K, G);
+        const uint8_t* gW[GEMV_GROUP_MAX];
+        float* gY[GEMV_GROUP_MAX];
+        int64_t gN[GEMV_GROUP_MAX], gL[GEMV_GROUP_MAX];
+        int n = 0;
+        for (int j = i; j < count; ++j) {
+            if (done[j] || gm_waves(N[j], K, G) != waves) continue;
+            gW[n] = W[j];
+            gY[n] = Y[j];
+            gN[n] = N[j];
+            gL[n] = ldy_m[j];
+            ++n;
+            done[j] = true;
+        }
+        const hipError_t e = launch_gm_waves(n, gW, gY, gN, gL, aqs, ads, K, M, ldy_n, dbg, waves, stream);
+        if (e != hipSuccess) return e;
     }
-    return waves == 16 ? launch_gm<16>(grp, wgs, aqs, ads, K, M, ldy_n, dbg, stream)
-                       : launch_gm<8>(grp, wgs, aqs, ads, K, M, ldy_n, dbg, stream);
+    return hipSuccess;
 }
-
-int gemv_mfma_waves(int64_t N) { return gm_plan(N).waves; }
 
 hipError_t launch_gemv_mfma(const uint8_t* W, const int8_t* aqs, const uint32_t* ads, float* Y, int64_t K,
                             int64_t N, int64_t M, int64_t ldy_m, int64_t ldy_n, int32_t* dbg, hipStream_t stream) {

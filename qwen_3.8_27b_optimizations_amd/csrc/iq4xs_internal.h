@@ -39,29 +39,27 @@ hipError_t launch_planar_to_blocks(const int8_t* qs, const uint32_t* ds, int64_t
 hipError_t launch_gemv(const uint8_t* W, const int8_t* aqs, const uint32_t* ads, float* Y, int64_t K, int64_t N,
                        int64_t M, int64_t ldy_m, int64_t ldy_n, int32_t* dbg, hipStream_t stream);
 
-// Small-batch GEMV on the int8 matrix cores (1 <= M <= 8, same contract as
-// launch_gemv); hipErrorNotSupported when the shape does not fit its LDS.
+// Small-batch multiply on the int8 matrix cores (1 <= M <= GM_MAX_COLS, same
+// contract as launch_gemv); hipErrorNotSupported past its 32-bit offsets.
+constexpr int64_t GM_MAX_COLS = 64;
 hipError_t launch_gemv_mfma(const uint8_t* W, const int8_t* aqs, const uint32_t* ads, float* Y, int64_t K,
                             int64_t N, int64_t M, int64_t ldy_m, int64_t ldy_n, int32_t* dbg, hipStream_t stream);
 
 // Matrices run together by one grouped GEMV launch (same K, same activations).
 constexpr int GEMV_GROUP_MAX = 4;
 
-// The matrix-core GEMV over count <= GEMV_GROUP_MAX matrices in one launch
-// (Y[i] element (m, n) at Y[i][m*ldy_m[i] + n*ldy_n]); every matrix must take
-// the same wave count (gemv_mfma_waves), else hipErrorNotSupported.  dbg only
-// with count == 1.  Outputs are bit-identical to one launch per matrix.
+// The matrix-core GEMV over count <= GEMV_GROUP_MAX matrices, one launch per
+// wave count (which follows each matrix's own shape)
+// (Y[i] element (m, n) at Y[i][m*ldy_m[i] + n*ldy_n]).  dbg only with
+// count == 1.  Outputs are bit-identical to one launch per matrix.
 hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
                                   const int64_t* ldy_m, const int8_t* aqs, const uint32_t* ads, int64_t K,
                                   int64_t M, int64_t ldy_n, int32_t* dbg, hipStream_t stream);
-// Waves per workgroup the matrix-core GEMV gives an N-row matrix (its rows'
-// summation order); matrices with equal counts can share a launch.
-int gemv_mfma_waves(int64_t N);
 
 // Y[i] = W[i] x for i < count <= GEMV_GROUP_MAX, M <= GEMV_MAX_COLS columns
 // of planar Q8_1 activations; Y[i] in ggml layout [M][N[i]] (layout_mk) or
-// [N[i]][M].  The matrices that launch_gemv runs on the matrix cores share a
-// launch per wave count, the others one tile-kernel launch (one launch per
+// [N[i]][M].  The matrices that launch_gemv runs on the matrix cores share its
+// launches, the others one tile-kernel launch (one launch per
 // matrix where the tile kernel does not take the shape); outputs are
 // bit-identical to launch_gemv on each matrix.
 hipError_t launch_gemv_group(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
