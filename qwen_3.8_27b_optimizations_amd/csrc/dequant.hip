@@ -8,53 +8,66 @@
 // outputs are bit-identical to the reference's CPU dequantiser.
 //
 // MI355X mapping.  The op moves 136 bytes in and 1024 bytes out per
-// super-block: it is bound by HBM writes.  Each thread takes 8 qs bytes of a
-// sub-block (16 codes: outputs 8 consecutive low-nibble weights and the 8
-// matching high-nibble weights) and writes them as four 16-byte stores, so a
-// wave writes 2 KB of contiguous output per store instruction pair; 16 threads
-// share a super-block and read its 8-byte header.  Codes are decoded with the
-// same v_perm lookup as the GEMV/GEMM (decode_codes_x).
+// super-block: it is bound by HBM writes, so every store instruction writes
+// whole 128-byte lines.  8 lanes share a pair of sub-blocks (2g, 2g + 1): lane
+// c (+ 4) takes qs dword c of both, the low (high) nibbles, so one 16-byte
+// store of the 8 lanes is sub-block 2g in output order and the next 2g + 1;
+// 32 threads share a super-block and read its 8-byte header.  (One lane for
+// both nibbles wrote 16-byte pieces 32 bytes apart: 5.2 against 5.8 TB/s on
+// 5120 x 17408, 78 against 70 us.)  Codes are decoded with the GEMV's v_perm
+// tables (decode_codes_x), one nibble at a time.
+//
+// An output too large to stay in the 256 MB Infinity Cache is written with
+// nontemporal stores, which measured 59 us = 6.8 TB/s there (a device fill
+// reaches 6.9); smaller ones with plain stores, as fast up to 192 MiB (34.2
+// against 33.4 us) and left in the cache for their reader.
 #include "iq4xs_device.h"
 #include "iq4xs_internal.h"
 
 namespace iq4xs {
 
+template <bool kStream>
 __global__ __launch_bounds__(256) void dequant_iq4xs_kernel(const uint8_t* __restrict__ src, float* __restrict__ dst,
                                                             int64_t n_blocks) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t b = t >> 4;
+    const int64_t b = t >> 5;
     if (b >= n_blocks) return;
-    const int p = (int)(t & 15);
-    const int ib = p >> 1, h = p & 1;  // sub-block, half (qs bytes 8h .. 8h+7 of the sub-block)
+    const int p = (int)(t & 31), g = p >> 3, c = p & 3, shift = p & 4;  // sub-block pair, qs dword, nibble
     const uint8_t* blk = src + b * BLOCK_BYTES;
     const v2u hd = *reinterpret_cast<const v2u*>(blk);
-    const v2u q = *reinterpret_cast<const v2u*>(blk + 8 + 16 * ib + 8 * h);
-    const float dl = half_bits_to_float(hd.x & 0xFFFFu) * (float)(subblock_ls(hd.x, hd.y, ib) - 32);
-    uint32_t lo[2], hi[2];
-    decode_codes_x(q.x, lo[0], hi[0]);
-    decode_codes_x(q.y, lo[1], hi[1]);
-    float* y = dst + b * QK_K + 32 * ib + 8 * h;
-    v4f out[4];
+    const uint32_t q0 = *reinterpret_cast<const uint32_t*>(blk + 8 + 32 * g + 4 * c);
+    const uint32_t q1 = *reinterpret_cast<const uint32_t*>(blk + 24 + 32 * g + 4 * c);
+    const float d = half_bits_to_float(hd.x & 0xFFFFu);
+    const float d0 = d * (float)(subblock_ls(hd.x, hd.y, 2 * g) - 32);
+    const float d1 = d * (float)(subblock_ls(hd.x, hd.y, 2 * g + 1) - 32);
+    const uint32_t k0 = decode_nibbles_x((q0 >> shift) & 0x0F0F0F0Fu);
+    const uint32_t k1 = decode_nibbles_x((q1 >> shift) & 0x0F0F0F0Fu);
+    v4f y0, y1;
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            out[w][k] = dl * (float)(int8_t)(lo[w] >> (8 * k));
-            out[2 + w][k] = dl * (float)(int8_t)(hi[w] >> (8 * k));
-        }
+    for (int k = 0; k < 4; ++k) {
+        y0[k] = d0 * (float)(int8_t)(k0 >> (8 * k));
+        y1[k] = d1 * (float)(int8_t)(k1 >> (8 * k));
     }
-    reinterpret_cast<v4f*>(y)[0] = out[0];
-    reinterpret_cast<v4f*>(y)[1] = out[1];
-    reinterpret_cast<v4f*>(y + 16)[0] = out[2];
-    reinterpret_cast<v4f*>(y + 16)[1] = out[3];
+    v4f* y = reinterpret_cast<v4f*>(dst + b * QK_K + 64 * g) + (p & 7);
+    if constexpr (kStream) {
+        __builtin_nontemporal_store(y0, y);
+        __builtin_nontemporal_store(y1, y + 8);
+    } else {
+        y[0] = y0;
+        y[8] = y1;
+    }
 }
 
 hipError_t launch_dequant(const uint8_t* src, float* dst, int64_t n_blocks, hipStream_t stream) {
     clear_launch_error();
-    const int64_t threads = n_blocks * 16;
+    const int64_t threads = n_blocks * 32;
     const int64_t grid = (threads + 255) / 256;
     if (grid > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(dequant_iq4xs_kernel, dim3((unsigned)grid), dim3(256), 0, stream, src, dst, n_blocks);
+    constexpr int64_t kCached = 192 * 1024;  // super-blocks of 1 KB of output: 192 MiB
+    if (n_blocks > kCached)
+        hipLaunchKernelGGL(dequant_iq4xs_kernel<true>, dim3((unsigned)grid), dim3(256), 0, stream, src, dst, n_blocks);
+    else
+        hipLaunchKernelGGL(dequant_iq4xs_kernel<false>, dim3((unsigned)grid), dim3(256), 0, stream, src, dst, n_blocks);
     return hipGetLastError();
 }
 

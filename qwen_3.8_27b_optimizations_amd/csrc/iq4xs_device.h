@@ -137,6 +137,11 @@ __device__ inline int dot4(uint32_t a, uint32_t b, int c) {
 constexpr uint32_t KXA0 = 0x40529881u, KXA1 = 0x091522cfu;
 constexpr uint32_t KXB0 = 0x26190dfeu, KXB1 = 0x8ea6ba35u;
 
+// Four codes, one per byte (0-15) -> four int8 codebook values.
+__device__ inline uint32_t decode_nibbles_x(uint32_t n) {
+    return __builtin_amdgcn_perm(KXA1, KXA0, n) ^ __builtin_amdgcn_perm(KXB1, KXB0, n ^ 0x08080808u);
+}
+
 __device__ inline void decode_codes_x(uint32_t q, uint32_t& lo, uint32_t& hi) {
     const uint32_t nl = q & 0x0F0F0F0Fu;
     const uint32_t xl = (q ^ 0x08080808u) & 0x0F0F0F0Fu;
