@@ -747,22 +747,19 @@ static bool f16_fits(int64_t K) {
     return (int64_t)H_BN * (K / QK_K) * BLOCK_BYTES < (1ll << 32) && (int64_t)H_BM * 2 * K < (1ll << 32);
 }
 
-// Token counts of the GEMM entry that the small-batch kernel takes: all up to
-// one of its token blocks, where the GEMM's tiles leave most of the chip idle
-// (us, GEMM against small-batch: gate + up M = 16 69 / 35, M = 32 77 / 54;
-// 17408 -> 5120 M = 16 79 / 22, M = 32 79 / 32; q/k/v M = 32 34 / 26), and two
-// blocks for matrices too narrow for the GEMM to fill it (M = 64: 17408 ->
-// 5120 79 / 57, 8192 -> 5120 41 / 32, but gate + up 77 / 88, q/k/v 34 / 36).
-// Below 2048 rows (k, v) a matrix stays with the q it is grouped with.
-static bool use_gemv_mfma_above_gemv(int64_t N, int64_t M) {
-    return M > GEMV_MAX_COLS && (M <= 32 || (M <= GM_MAX_COLS && N >= 2048 && N < 8192));
-}
+// Token counts of the GEMM entry that the small-batch kernel takes: all of its
+// range, where the GEMM's 128-row tiles leave much of the chip idle or unfed
+// (us, GEMM against small-batch: gate + up M = 16 69 / 37, M = 32 77 / 47, M =
+// 64 77 / 70; 17408 -> 5120 79 / 22, 79 / 29, 79 / 44; 8192 -> 5120 M = 33
+// 41 / 20; q/k/v M = 64 34 / 33; the one loss is a single 17408-row matrix from
+// M = 57 on, 43 / 45.5, whose pair gains as much).
+static bool use_gemv_mfma_above_gemv(int64_t M) { return M > GEMV_MAX_COLS && M <= GM_MAX_COLS; }
 
 hipError_t launch_gemm(const uint8_t* W, const int8_t* aqs, const uint32_t* ads, const uint32_t* ahq, float* Y,
                        int64_t K, int64_t N, int64_t M, int64_t ldy_m, int64_t ldy_n, int32_t* dbg,
                        hipStream_t stream) {
     clear_launch_error();
-    if (use_gemv_mfma_above_gemv(N, M)) {
+    if (use_gemv_mfma_above_gemv(M)) {
         const hipError_t e = launch_gemv_mfma(W, aqs, ads, Y, K, N, M, ldy_m, ldy_n, dbg, stream);
         if (e != hipErrorNotSupported) return e;
     }
@@ -787,45 +784,24 @@ hipError_t launch_gemm_group(int count, const uint8_t* const* W, float* const* Y
                              hipStream_t stream) {
     clear_launch_error();
     if (count < 1 || count > GEMV_GROUP_MAX) return hipErrorInvalidValue;
-    // the small-batch kernel's matrices first (the same routing as single calls)
     const int64_t ldy_n = layout_mk ? 1 : M;
-    const uint8_t *gW[GEMV_GROUP_MAX], *sW[GEMV_GROUP_MAX];
-    float *gY[GEMV_GROUP_MAX], *sY[GEMV_GROUP_MAX];
-    int64_t gN[GEMV_GROUP_MAX], sN[GEMV_GROUP_MAX], sL[GEMV_GROUP_MAX];
-    int n = 0, ns = 0;
-    for (int i = 0; i < count; ++i) {
-        if (use_gemv_mfma_above_gemv(N[i], M)) {
-            sW[ns] = W[i];
-            sY[ns] = Y[i];
-            sN[ns] = N[i];
-            sL[ns++] = layout_mk ? N[i] : 1;
-        } else {
-            gW[n] = W[i];
-            gY[n] = Y[i];
-            gN[n++] = N[i];
-        }
+    if (use_gemv_mfma_above_gemv(M)) {
+        int64_t ldy_m[GEMV_GROUP_MAX];
+        for (int i = 0; i < count; ++i) ldy_m[i] = layout_mk ? N[i] : 1;
+        const hipError_t e = launch_gemv_mfma_group(count, W, Y, N, ldy_m, aqs, ads, K, M, ldy_n, nullptr, stream);
+        if (e != hipErrorNotSupported) return e;
     }
-    if (ns > 0) {
-        const hipError_t e = launch_gemv_mfma_group(ns, sW, sY, sN, sL, aqs, ads, K, M, ldy_n, nullptr, stream);
-        if (e == hipErrorNotSupported) {  // shapes past its offsets
-            n = count;
-            for (int i = 0; i < count; ++i) gW[i] = W[i], gY[i] = Y[i], gN[i] = N[i];
-        } else if (e != hipSuccess) {
-            return e;
-        }
-    }
-    if (n == 0) return hipSuccess;
     if (!f16_fits(K)) return hipErrorInvalidConfiguration;
     GemmGroup grp{};
     int64_t tiles = 0;
     for (int i = 0; i < GEMV_GROUP_MAX; ++i) {
-        const int j = i < n ? i : n - 1;  // unused entries repeat the last matrix, past every tile
-        if (i < n) tiles += (gN[j] + H_BN - 1) / H_BN;
+        const int j = i < count ? i : count - 1;  // unused entries repeat the last matrix, past every tile
+        if (i < count) tiles += (N[j] + H_BN - 1) / H_BN;
         if (tiles > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
-        grp.W[i] = gW[j];
-        grp.Y[i] = gY[j];
-        grp.N[i] = gN[j];
-        grp.ldy_m[i] = layout_mk ? gN[j] : 1;
+        grp.W[i] = W[j];
+        grp.Y[i] = Y[j];
+        grp.N[i] = N[j];
+        grp.ldy_m[i] = layout_mk ? N[j] : 1;
         grp.tile_end[i] = (int)tiles;
     }
     return launch_f16_kernel<false, true>(grp, tiles, aqs, ahq, ads, K, M, layout_mk ? 1 : M, nullptr, stream);

@@ -9,13 +9,13 @@
 // Why a second GEMV.  The dot4 GEMV spends VALU work per weight byte and per
 // column, so from 4 columns on it is VALU-bound.  Here one
 // v_mfma_i32_32x32x32_i8 takes 32 weight rows x 32 k of one sub-block against
-// up to 32 columns (the A operand is the activations, one token per MFMA row;
+// 32 columns (the A operand is the activations, one token per MFMA row;
 // rows past M hold any token and only produce C rows that are never stored),
 // so the VALU cost is the decode of the codes into the B operand, the same for
 // any M, and per output a subtract, a scale product and a fused add.
 //
 // Mapping.  A workgroup owns up to 32 weight rows (one MFMA block) of one
-// matrix and 8 G tokens, and splits K over its waves: wave w takes the
+// matrix and all columns (8 G of them), and splits K over its waves: wave w takes the
 // super-blocks kb = w, w + waves, ... (at any moment the waves stream adjacent
 // super-blocks of the same rows), with no barrier before the final sum.  The
 // partial sums are added in wave order and the wave count follows the
@@ -33,7 +33,9 @@
 //     nibbles of qs bytes 8h .. 8h+7 of the sub-block (weights 8h .. 8h+7 and
 //     16+8h .. 16+8h+7), and the A lanes the activation codes of the same 16
 //     weights, which the staging puts side by side (one 16-byte read).
-//   * The C element e of lane l is token 8*(e>>2) + 4h + (e&3) of its row.
+//   * The C element e of lane l is token 8*(e>>2) + 4h + (e&3) of its row; past
+//     32 columns a second MFMA takes the same B operand, so the decode is not
+//     repeated.
 //   * The int32 sum comes back as a float without a convert (which issues at
 //     half the rate of an add): the accumulator starts at the bits of
 //     1/(2 pi) = 0x3E22F983, an inline constant in the middle of the binade
@@ -48,18 +50,24 @@ namespace iq4xs {
 
 constexpr int GM_LDS_MAX = 160 * 1024;
 
-constexpr int GM_AROW = 272;  // LDS row of one token's 256 codes, padded (conflict-free 16-byte reads)
+// Activations are staged a whole super-block at a time up to 16 tokens, above
+// in halves of 4 sub-blocks: less LDS and fewer registers in flight, hence
+// more waves per CU.
+constexpr int gm_halves(int G) { return G <= 2 ? 1 : 2; }
+// LDS row of one token's staged codes, padded (conflict-free 16-byte reads)
+constexpr int gm_arow(int G) { return QK_K / gm_halves(G) + 16; }
 constexpr int GM_WROW = 136;  // LDS row of one weight row's 128 qs bytes, padded (conflict-free 8-byte reads)
 // per-wave staging bytes: weight rows, token rows, then the super-block's
 // column scales [8 sub-blocks][8G tokens]; the final sum reuses them
-constexpr int gm_wave_lds(int G) { return 32 * GM_WROW + G * (8 * GM_AROW + 8 * 8 * 4); }
+constexpr int gm_wave_lds(int G) { return 32 * GM_WROW + G * (8 * gm_arow(G) + 8 * 8 * 4); }
 
 constexpr int GM_ZERO_BITS = 0x3E22F983;  // the accumulator's zero (1/(2 pi) as a float)
 
 // Most waves of a workgroup (gm_waves).
-constexpr int gm_max_waves(int G) { return G <= 2 ? 16 : 8; }
-// Waves per SIMD that the registers are held to (96, 114, 146 and 152 VGPRs).
-constexpr int gm_waves_per_simd(int G, bool debug) { return G == 1 ? 5 : (G == 2 ? 4 : (debug ? 2 : 3)); }
+constexpr int gm_max_waves(int G) { return G == 1 ? 16 : G <= 6 ? 12 : 8; }
+// Waves per SIMD that the registers are held to (96 to 128 VGPRs up to G = 4,
+// 161 and 168 at 5 and 6, 226 and 246 at 7 and 8, where the LDS allows no more).
+constexpr int gm_waves_per_simd(int G, bool debug) { return G == 1 ? 5 : (G == 2 ? 4 : (debug || G > 6 ? 2 : G <= 4 ? 4 : 3)); }
 
 // The matrices of one launch (same K and activations): workgroups
 // [tile_end[i-1], tile_end[i]) run matrix i.  Entries past the group's count
@@ -76,11 +84,12 @@ struct GmGroup {
 template <int G, bool kDebug>
 __global__ __launch_bounds__(64 * gm_max_waves(G)) __attribute__((amdgpu_waves_per_eu(gm_waves_per_simd(G, kDebug))))
 void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const uint32_t* __restrict__ ads, int K,
-                      int M, int rows, int toks, int64_t ldy_n, int32_t* __restrict__ dbg) {
-    // sub-blocks unrolled together: all 8, fewer where the registers of their
-    // reads in flight would cost a wave per SIMD (M = 32, gate + up: 2 together
-    // 56.6 us, 1 at a time 50.6)
-    constexpr int UNR = kDebug || G == 4 ? 1 : (G == 3 ? 2 : 8);
+                      int M, int rows, int64_t ldy_n, int32_t* __restrict__ dbg) {
+    // sub-blocks unrolled together: above 16 tokens one at a time, since the
+    // registers of more reads in flight would cost waves (M = 32, gate + up: 2
+    // together 56.6 us, 1 at a time 50.6)
+    constexpr int UNR = kDebug || G >= 3 ? 1 : 8;
+    constexpr int HALVES = gm_halves(G), SUB = 8 / HALVES, AROW = gm_arow(G);
     extern __shared__ __attribute__((aligned(16))) uint8_t gm_lds[];
     // this workgroup's matrix: scalar selects on the by-value descriptor (a
     // dynamic index into it would go through scratch)
@@ -102,19 +111,15 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, col = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = (int)blockDim.x >> 6;
     uint8_t* sw = gm_lds + wave * gm_wave_lds(G);                   // [32][136] qs of a block's rows
-    uint8_t* sact = sw + 32 * GM_WROW;                              // [8G][272] activations
-    float* sdx = reinterpret_cast<float*>(sact + 8 * G * GM_AROW);  // [8][8G] column scales (0 past M)
+    uint8_t* sact = sw + 32 * GM_WROW;                              // [8G][AROW] activations
+    float* sdx = reinterpret_cast<float*>(sact + 8 * G * AROW);  // [8][8G] column scales (0 past M)
     const int r0 = ((int)blockIdx.x - tile0) * rows;
     const int nrow = min(rows, N - r0);  // this workgroup's rows (1 .. 32)
-    const int t0 = (int)blockIdx.y * toks;
-    const int mt = min(toks, M - t0);  // this workgroup's tokens (1 .. 8G)
     // Global loads are 32-bit lane offsets from workgroup-uniform bases.  MFMA
     // rows past nrow are clamped to its last row (a repeat of bytes already
     // loaded, so no extra HBM traffic): computed, never stored.
     const uint32_t row_bytes = (uint32_t)bpr * BLOCK_BYTES;
     const uint8_t* wbase = W + (size_t)r0 * row_bytes;
-    const int8_t* abase = aqs + (size_t)t0 * K;
-    const uint32_t* dbase = ads + (size_t)t0 * nb;
 
     // an offset kept scalar: the loads then take a scalar base and a 32-bit
     // lane offset, instead of a 64-bit address per lane and load
@@ -124,7 +129,8 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
     };
     v2u wh;        // d, scales_h, scales_l of row col
     v4i wq[4];     // qs chunk lane % 8 of rows lane/8 + 8i
-    v4i xa[G][2];  // sub-block lane % 8 of token 8g + lane/8
+    // sub-block lane % 8 of token 8g + lane/8, or of a half the 16 codes lane % 8 of it
+    v4i xa[G][2 / HALVES];
     uint32_t xd[G];
     auto load_w = [&](int kb) {
         const uint8_t* wk = wbase + uniform(kb * BLOCK_BYTES);
@@ -134,34 +140,39 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
             wq[i] = *reinterpret_cast<const v4i_a8*>(
                 wk + ((uint32_t)min(8 * i + (lane >> 3), nrow - 1) * row_bytes + 8 + 16 * (lane & 7)));
     };
-    auto load_x = [&](int kb) {
-        const int8_t* ak = abase + uniform(kb * QK_K);
-        const uint32_t* dk = dbase + uniform(kb * 8);
+    auto load_x = [&](int kb, int half) {
+        const int8_t* ak = aqs + uniform(kb * QK_K + half * 128);
+        const uint32_t* dk = ads + uniform(kb * 8);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            const uint32_t t = (uint32_t)min(8 * g + (lane >> 3), mt - 1);
-            const uint32_t off = t * (uint32_t)K + 32 * (lane & 7);
-            xa[g][0] = *reinterpret_cast<const v4i*>(ak + off);
-            xa[g][1] = *reinterpret_cast<const v4i*>(ak + off + 16);
-            xd[g] = dk[t * (uint32_t)nb + (lane & 7)];
+            const uint32_t t = (uint32_t)min(8 * g + (lane >> 3), M - 1);
+            const uint32_t off = t * (uint32_t)K + (32 / HALVES) * (lane & 7);
+#pragma unroll
+            for (int i = 0; i < 2 / HALVES; ++i) xa[g][i] = *reinterpret_cast<const v4i*>(ak + off + 16 * i);
+            if (half == 0) xd[g] = dk[t * (uint32_t)nb + (lane & 7)];
         }
     };
     // LDS operations of one wave complete in order: the reads below by other
     // lanes of the wave see these writes, and the previous block's reads were
     // issued before them
-    uint8_t* xwrite = sact + (lane >> 3) * GM_AROW + 32 * (lane & 7);
-    const uint8_t* xread = sact + min(col, 8 * G - 1) * GM_AROW + 16 * h;
+    uint8_t* xwrite = sact + (lane >> 3) * AROW + (HALVES == 1 ? 32 * (lane & 7) : 32 * ((lane & 7) >> 1) + 8 * (lane & 1));
+    const uint8_t* xread = sact + min(col, 8 * G - 1) * AROW + 16 * h;
     uint8_t* wwrite = sw + (lane >> 3) * GM_WROW + 16 * (lane & 7);
     const uint8_t* wread = sw + col * GM_WROW + 8 * h;
-    auto stage_x = [&]() {
+    auto stage_x = [&](int half) {
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            // elements 0-7, 16-23 and 8-15, 24-31: the A operand of each lane half
-            *reinterpret_cast<v4i*>(xwrite + 8 * g * GM_AROW) = v4i{xa[g][0].x, xa[g][0].y, xa[g][1].x, xa[g][1].y};
-            *reinterpret_cast<v4i*>(xwrite + 8 * g * GM_AROW + 16) =
-                v4i{xa[g][0].z, xa[g][0].w, xa[g][1].z, xa[g][1].w};
+            // a sub-block's elements in the order 0-7, 16-23, 8-15, 24-31: the A operand of each lane half
+            uint8_t* x = xwrite + 8 * g * AROW;
+            if constexpr (HALVES == 1) {
+                *reinterpret_cast<v4i*>(x) = v4i{xa[g][0].x, xa[g][0].y, xa[g][1].x, xa[g][1].y};
+                *reinterpret_cast<v4i*>(x + 16) = v4i{xa[g][0].z, xa[g][0].w, xa[g][1].z, xa[g][1].w};
+            } else {
+                *reinterpret_cast<v2u*>(x) = v2u{(uint32_t)xa[g][0].x, (uint32_t)xa[g][0].y};
+                *reinterpret_cast<v2u*>(x + 16) = v2u{(uint32_t)xa[g][0].z, (uint32_t)xa[g][0].w};
+            }
             const int t = 8 * g + (lane >> 3);
-            sdx[(lane & 7) * 8 * G + t] = t < mt ? half_bits_to_float(xd[g] & 0xFFFFu) : 0.0f;
+            if (half == 0) sdx[(lane & 7) * 8 * G + t] = t < M ? half_bits_to_float(xd[g] & 0xFFFFu) : 0.0f;
         }
     };
     auto stage_w = [&]() {
@@ -175,35 +186,40 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
     float acc[4 * G];
 #pragma unroll
     for (int e = 0; e < 4 * G; ++e) acc[e] = 0.0f;
-    auto compute = [&](const v2u hd, int kb) {
+    auto compute = [&](const v2u hd, int kb, int half) {
         const float dw = half_bits_to_float(hd.x & 0xFFFFu) * 67108864.0f;  // 2^26
 #pragma unroll UNR
-        for (int s = 0; s < 8; ++s) {
+        for (int i = 0; i < SUB; ++i) {
+            const int s = SUB * half + i;
             uint32_t lo0, hi0, lo1, hi1;
             const v2u q = *reinterpret_cast<const v2u*>(wread + 16 * s);
             decode_codes_x(q.x, lo0, hi0);
             decode_codes_x(q.y, lo1, hi1);
             const v4i bw = v4i{(int)lo0, (int)lo1, (int)hi0, (int)hi1};
-            const v4i ax = *reinterpret_cast<const v4i*>(xread + 32 * s);
             v16i z;
 #pragma unroll
             for (int e = 0; e < 16; ++e) z[e] = GM_ZERO_BITS;
-            const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(ax, bw, z, 0, 0, 0);
             const int ls = subblock_ls(hd.x, hd.y, s) - 32;
             const float sa = dw * (float)ls;
+            // 32 tokens (4 groups of 8) per MFMA
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const v4f bx = *reinterpret_cast<const v4f*>(sdx + s * 8 * G + 8 * g + 4 * h);
+            for (int b = 0; b < (G + 3) / 4; ++b) {
+                const uint8_t* xr = b == 0 ? xread : sact + min(32 * b + col, 8 * G - 1) * AROW + 16 * h;
+                const v4i ax = *reinterpret_cast<const v4i*>(xr + 32 * i);
+                const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(ax, bw, z, 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int e = 4 * g + j;
-                    const float f = __builtin_bit_cast(float, (int)c[e]) - __builtin_bit_cast(float, GM_ZERO_BITS);
-                    acc[e] = __builtin_fmaf(f, sa * bx[j], acc[e]);
-                    if (kDebug) {
-                        const int t = 8 * g + 4 * h + j;
-                        if (t < mt && col < nrow)
-                            dbg[((size_t)(t0 + t) * N + r0 + col) * nb + kb * 8 + s] =
-                                ((int)c[e] - GM_ZERO_BITS) * ls;
+                for (int g = 4 * b; g < (4 * b + 4 < G ? 4 * b + 4 : G); ++g) {
+                    const v4f bx = *reinterpret_cast<const v4f*>(sdx + s * 8 * G + 8 * g + 4 * h);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int e = 4 * g + j, ce = (int)c[e - 16 * b];
+                        const float f = __builtin_bit_cast(float, ce) - __builtin_bit_cast(float, GM_ZERO_BITS);
+                        acc[e] = __builtin_fmaf(f, sa * bx[j], acc[e]);
+                        if (kDebug) {
+                            const int t = 8 * g + 4 * h + j;
+                            if (t < M && col < nrow)
+                                dbg[((size_t)t * N + r0 + col) * nb + kb * 8 + s] = (ce - GM_ZERO_BITS) * ls;
+                        }
                     }
                 }
             }
@@ -211,16 +227,21 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
     };
     // every load is unconditional (past this wave's last super-block it repeats that one)
     if (wave < bpr) {
-        load_x(wave);
+        load_x(wave, 0);
         load_w(wave);
         for (int kb = wave; kb < bpr; kb += waves) {
             const int kn = kb + waves < bpr ? kb + waves : kb;
             const v2u hd = wh;
-            stage_x();
-            load_x(kn);
+            stage_x(0);
+            load_x(HALVES == 1 ? kn : kb, HALVES - 1);
             stage_w();
             load_w(kn);
-            compute(hd, kb);
+            compute(hd, kb, 0);
+            if constexpr (HALVES == 2) {
+                stage_x(1);
+                load_x(kn, 0);
+                compute(hd, kb, 1);
+            }
         }
     }
     // the waves' partial sums, added in wave order
@@ -235,33 +256,32 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
         float v = red[e * 64 + lane];
         for (int w = 1; w < waves; ++w) v += red[w * PER + e * 64 + lane];
         const int t = 8 * (e >> 2) + 4 * h + (e & 3);
-        if (t < mt && col < nrow) Y[(int64_t)(t0 + t) * ldy_m + (int64_t)(r0 + col) * ldy_n] = v;
+        if (t < M && col < nrow) Y[(int64_t)t * ldy_m + (int64_t)(r0 + col) * ldy_n] = v;
     }
 }
-
-// Tokens: blocks of at most 32, as even as possible.
-static int64_t gm_token_blocks(int64_t M) { return (M + 31) / 32; }
-static int64_t gm_tokens(int64_t M) { return (M + gm_token_blocks(M) - 1) / gm_token_blocks(M); }
 
 // Waves per workgroup of an N-row matrix.  They fix a row's fp32 summation
 // order, so they follow the matrix's own shape and M, never the launch.
 //   * From 384 row blocks on (gate/up, N = 17408) the blocks alone nearly fill
-//     the chip: 8 waves each, 4 past 16 tokens, where the registers allow 12
-//     waves per CU.  Below, K is split further so that every CU has loads in
-//     flight: 12 waves, 16 from K = 8192 on (as fast, with shorter sums), or 8
-//     past 16 tokens.  Measured (us per launch, 4 / 8 /
-//     12 waves): gate + up M = 8 30.6 / 30.3 / 33.4, M = 32 54.3 / 63.6 / 68.9;
-//     17408 -> 5120 M = 8 32.5 / 21.0 / 18.7 (16 waves: 19.1), M = 32 48.7 / 32.0 / 33.5; q/k/v
-//     M = 16 16.8 / 16.4 / 17.4.
+//     the chip: 8 waves each, 4 past 32 tokens, where a workgroup of 8 leaves
+//     no room for a second one.
+//   * Below, K is split further so that every CU has loads in flight: 12
+//     waves, 8 past 48 tokens (all that the LDS holds), 16 up to 8 tokens from
+//     K = 8192 on (as fast, with shorter sums).
+// Measured, us per launch with 4 / 8 / 12 waves: gate + up M = 8 30.6 / 30.3 /
+// 33.4, M = 32 48.5 / 47.7 / 55.2, M = 33 55 / 75 / 70, M = 64 70 / 81; 17408
+// -> 5120 M = 8 32.5 / 21.0 / 18.7 (16 waves 19.1), M = 32 50 / 33 / 29, M = 33
+// 66 / 43 / 36, M = 64 59 / 44; q/k/v M = 64 30 / 33.
 static int gm_waves(int64_t N, int64_t K, int G) {
     const int64_t bpr = K / QK_K;
-    const int w = (N + 31) / 32 >= 384 ? (G <= 2 ? 8 : 4) : (G <= 2 && bpr < 32 ? 12 : gm_max_waves(G));
+    const int narrow = G == 1 && bpr < 32 ? 12 : gm_max_waves(G);
+    const int w = (N + 31) / 32 >= 384 ? (G <= 4 ? 8 : 4) : narrow;
     return (int)std::max<int64_t>(4, std::min<int64_t>(w, bpr));
 }
 
 template <int G>
 static hipError_t launch_gm(const GmGroup& grp, dim3 grid, int waves, const int8_t* aqs, const uint32_t* ads,
-                            int64_t K, int64_t M, int64_t rows, int64_t toks, int64_t ldy_n, int32_t* dbg,
+                            int64_t K, int64_t M, int64_t rows, int64_t ldy_n, int32_t* dbg,
                             hipStream_t stream) {
     const size_t lds = (size_t)waves * gm_wave_lds(G);
     static_assert(gm_max_waves(G) * gm_wave_lds(G) <= GM_LDS_MAX, "the staging fits a CU");
@@ -272,7 +292,7 @@ static hipError_t launch_gm(const GmGroup& grp, dim3 grid, int waves, const int8
             if (e != hipSuccess) return e;
         }
         hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), lds, stream, grp, aqs, ads, (int)K, (int)M, (int)rows,
-                           (int)toks, ldy_n, dbg);
+                           ldy_n, dbg);
         return hipGetLastError();
     };
     return dbg ? launch(&gemv_mfma_kernel<G, true>) : launch(&gemv_mfma_kernel<G, false>);
@@ -282,14 +302,14 @@ static hipError_t launch_gm(const GmGroup& grp, dim3 grid, int waves, const int8
 static hipError_t launch_gm_waves(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
                                   const int64_t* ldy_m, const int8_t* aqs, const uint32_t* ads, int64_t K, int64_t M,
                                   int64_t ldy_n, int32_t* dbg, int waves, hipStream_t stream) {
-    const int64_t tblocks = gm_token_blocks(M), toks = gm_tokens(M), cus = device_cu_count();
+    const int64_t cus = device_cu_count();
     // Rows per workgroup: 32, fewer where that leaves CUs without one (N =
     // 5120: 20 rows on 256 CUs against 160 blocks of 32); at least 8, since
     // each workgroup decodes all 32 MFMA rows whatever it keeps (N = 1024, M =
     // 8: 6.6 us with 8 rows against 7.0 with 4).
     int64_t total = 0;
     for (int i = 0; i < count; ++i) total += N[i];
-    const int64_t rows = std::max<int64_t>(8, std::min<int64_t>(32, (total * tblocks + cus - 1) / cus));
+    const int64_t rows = std::max<int64_t>(8, std::min<int64_t>(32, (total + cus - 1) / cus));
     GmGroup grp{};
     int64_t wgs = 0;
     for (int i = 0; i < GEMV_GROUP_MAX; ++i) {
@@ -302,13 +322,21 @@ static hipError_t launch_gm_waves(int count, const uint8_t* const* W, float* con
         grp.N[i] = (int)N[j];
         grp.tile_end[i] = (int)wgs;
     }
-    const dim3 grid((unsigned)wgs, (unsigned)tblocks);
-    switch ((toks + 7) / 8) {
-        case 1: return launch_gm<1>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
-        case 2: return launch_gm<2>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
-        case 3: return launch_gm<3>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
-        default: return launch_gm<4>(grp, grid, waves, aqs, ads, K, M, rows, toks, ldy_n, dbg, stream);
+    const dim3 grid((unsigned)wgs);
+#define IQ4XS_GM(G) \
+    case G: return launch_gm<G>(grp, grid, waves, aqs, ads, K, M, rows, ldy_n, dbg, stream)
+    switch ((M + 7) / 8) {
+        IQ4XS_GM(1);
+        IQ4XS_GM(2);
+        IQ4XS_GM(3);
+        IQ4XS_GM(4);
+        IQ4XS_GM(5);
+        IQ4XS_GM(6);
+        IQ4XS_GM(7);
+        IQ4XS_GM(8);
+        default: return hipErrorNotSupported;
     }
+#undef IQ4XS_GM
 }
 
 hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
@@ -317,13 +345,13 @@ hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* con
     clear_launch_error();
     if (count < 1 || count > GEMV_GROUP_MAX || (dbg && count != 1)) return hipErrorInvalidValue;
     if (M < 1 || M > GM_MAX_COLS || K % QK_K || K >= (1 << 24)) return hipErrorNotSupported;
-    // the kernel's 32-bit load offsets span 32 rows and 32 tokens
-    if ((int64_t)32 * (K / QK_K) * BLOCK_BYTES >= ((int64_t)1 << 31) || (int64_t)32 * K >= ((int64_t)1 << 31))
+    // the kernel's 32-bit load offsets span 32 rows and GM_MAX_COLS tokens
+    if ((int64_t)32 * (K / QK_K) * BLOCK_BYTES >= ((int64_t)1 << 31) || GM_MAX_COLS * K >= ((int64_t)1 << 31))
         return hipErrorNotSupported;
     for (int i = 0; i < count; ++i)
         if (N[i] < 1 || N[i] >= (1 << 30)) return hipErrorNotSupported;
     // one launch per wave count
-    const int G = (int)((gm_tokens(M) + 7) / 8);
+    const int G = (int)((M + 7) / 8);
     bool done[GEMV_GROUP_MAX] = {};
     for (int i = 0; i < count; ++i) {
         if (done[i]) continue;

@@ -10,12 +10,13 @@ from oracle.oracle import LAYOUT_KM, LAYOUT_MK, compute_metrics
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
-# K, N, M: the first and last M of each 8-token step, one to 32 tokens and the two-block range; a row
+# K, N, M: the first and last M of each 8-token step (two MFMAs per decode past 32); a row
 # block of 1, 20 and 32 rows and a ragged last one; one super-block, fewer than the waves, and a K whose
 # super-blocks do not divide among them; both sides of 384 row blocks
 CASES = [(256, 1, 9), (256, 33, 16), (768, 70, 17), (2048, 95, 24), (2304, 64, 25), (5120, 129, 32),
          (8448, 40, 16), (768, 5120 + 7, 12), (512, 32 * 384, 10), (256, 32 * 383 - 5, 31), (512, 2048, 33),
-         (768, 2049, 48), (256, 8191, 49), (1280, 2100, 64)]
+         (768, 2049, 48), (256, 8191, 49), (1280, 2100, 64), (256, 32 * 384, 40), (768, 32 * 383 + 5, 41),
+         (3328, 90, 56), (5120, 33, 57), (512, 32 * 384 + 1, 64), (8192, 64, 8)]
 
 
 @pytest.mark.parametrize("K,N,M", CASES)
@@ -27,7 +28,7 @@ def test_token_and_row_blocks(pkg, orc, K, N, M):
     AQ = orc.quantize_q8_1_batched(X, K, M, LAYOUT_MK)
     Wd = torch.from_numpy(W).to(dev)
     ws = pkg.quantize_q8_1(torch.from_numpy(X).to(dev), K, M, LAYOUT_MK)
-    S, Yd = pkg.subblock_sums(Wd, ws, K, N, M, pkg.PATH_GEMM)
+    S, Yd = pkg.subblock_sums(Wd, ws, K, N, M, pkg.PATH_GEMM if M > 8 else pkg.PATH_GEMV)
     Y = pkg.mul_mat_q8_1(Wd, ws, K, N, M, LAYOUT_MK)
     Ykm = pkg.mul_mat_q8_1(Wd, ws, K, N, M, LAYOUT_KM)
     n2 = min(N, 100)  # a second matrix of another size in the same call
