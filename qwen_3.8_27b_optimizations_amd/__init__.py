@@ -125,16 +125,26 @@ def lib() -> Lib:
 # ---------------------------------------------------------------------------
 # torch helpers (device memory and streams only)
 
-def _torch():
-    import torch
+_TORCH = None  # the module, once a GPU has been seen
 
-    if not torch.cuda.is_available():
-        raise RuntimeError("no ROCm GPU visible: the IQ4_XS kernels have no CPU path")
-    return torch
+
+def _torch():
+    global _TORCH
+    if _TORCH is None:
+        import torch
+
+        if not torch.cuda.is_available():
+            raise RuntimeError("no ROCm GPU visible: the IQ4_XS kernels have no CPU path")
+        _TORCH = torch
+    return _TORCH
 
 
 def _stream(torch) -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle of torch.cuda.current_stream() without building the Stream
+    # object: with the availability check made once, 0.4 us of a call's host
+    # time against 3.6 (a one-column mul_mat 8.1 -> 5.5 us)
+    torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _check_weights(W, K: int, N: int) -> None:
