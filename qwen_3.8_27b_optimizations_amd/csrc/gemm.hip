@@ -172,15 +172,16 @@ struct HWeights {  // one super-block of this lane's weight row: header, and qs 
 };
 
 // One super-block of the fp16 kernel for one wave: the MFMAs and epilogue of
-// its 4 sub-blocks x 4 token blocks from stage `st` (tokens) and `w` (its
-// weight row), as a software pipeline over the 16 (sub-block, token block)
+// its 4 sub-blocks x 4 token blocks from `st` (tokens), `tst` (their scales)
+// and `w` (its weight row), as a software pipeline over the 16 (sub-block, token block)
 // steps: step t issues its three MFMAs, then the FMAs of step t - 1 (whose
 // results have landed meanwhile) while the LDS fragments of step t + 1 are in
 // flight; the next sub-block's weights are decoded during the current one.
 // `w` is reloaded with the next super-block (load_next) once its last
 // sub-block is decoded, so one set of weight registers serves both.
 template <bool kDebug, int T, int TOK, typename LoadNext>
-__device__ __forceinline__ void f16_superblock(const uint8_t* st, const uint8_t* lut, HWeights& w, v16f (&acc)[4],
+__device__ __forceinline__ void f16_superblock(const uint8_t* st, const uint8_t* tst, const uint8_t* lut, HWeights& w,
+                                               v16f (&acc)[4],
                                                int kh, int h, int col, int lane, int64_t kb, int64_t m0, int64_t M,
                                                int64_t n, int64_t N, int64_t nb, int32_t* __restrict__ dbg,
                                                LoadNext&& load_next) {
@@ -226,7 +227,7 @@ __device__ __forceinline__ void f16_superblock(const uint8_t* st, const uint8_t*
         if (r < 2)
             a = *reinterpret_cast<const v4u*>(st + h_chunk(m, 4 * s + 2 * h + r));
         else
-            a = *reinterpret_cast<const v4u*>(st + HStage<TOK>::t_off + h * HStage<TOK>::t_copy + m * 32 + 16 * kh);
+            a = *reinterpret_cast<const v4u*>(tst + h * HStage<TOK>::t_copy + m * 32 + 16 * kh);
     };
     // half q of the epilogue of step t: acc += sp * dp for accumulators 8q .. 8q + 7
     auto epilogue = [&](int t, const v16f& dp, const v16f& sp, int q) {
@@ -365,7 +366,13 @@ __device__ __forceinline__ void f16_tile(const uint8_t* __restrict__ W, float* _
                                          int by, uint8_t* smem, int32_t* __restrict__ dbg) {
     static_assert(RG == 4 || (RG == 2 && T <= 2), "half-height tiles hold at most 64 tokens");
     constexpr int TOK = 32 * RG, STAGE = HStage<TOK>::bytes;
-    constexpr int CPW = 8 * T / RG;  // 1 KB token copies per wave and stage (16 T per stage)
+    constexpr int CPW = 8 * T / RG;  // 1 KB token copies per wave and super-block (16 T in all)
+    // Super-blocks per stage: a stage holds TOK rows of a token and a
+    // super-block, so a 128-row tile of 32 tokens takes four super-blocks
+    // between two barriers, with its copies further ahead (17408 -> 5120 at M =
+    // 130: 98 -> 92 us).  Tiles of 64 tokens and half-height tiles measured
+    // 3-4 % slower with two.
+    constexpr int SB = T == 1 && RG == 4 ? 4 : 1;
     uint8_t(*const stages)[STAGE] = reinterpret_cast<uint8_t(*)[STAGE]>(smem + H_LUT);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in an SGPR
@@ -395,25 +402,30 @@ __device__ __forceinline__ void f16_tile(const uint8_t* __restrict__ W, float* _
     // for CPW = 2, 4, 8 the bits of xrow & 15 and of 2i are disjoint, so the
     // swizzled chunk is (col ^ (xrow & 15)) ^ 2i: one XOR per copy
     const uint32_t xcol = 16u * (uint32_t)(col ^ (xrow & 15));
-    auto issue_x = [&](int64_t kb, int stage) {
-        const uint8_t* src = xtile + kb * 512;
+    // super-block kb (the last one repeats) into slot i of a stage
+    auto issue_x = [&](int64_t kb, int stage, int slot) {
+        const uint8_t* src = xtile + min(kb, bpr - 1) * 512;
 #pragma unroll
         for (int i = 0; i < CPW; ++i) {
             const int m = xrow + 2 * i;
             const uint32_t c16 = (CPW & (CPW - 1)) ? 16u * (uint32_t)(col ^ (m & 15)) : (xcol ^ (32u * i));
-            dma16(src, (uint32_t)min(m, xlast) * xstride + c16, lds_wave + stage * STAGE + i * 1024);
+            dma16(src, (uint32_t)min(m, xlast) * xstride + c16,
+                  lds_wave + stage * STAGE + slot * (32 * T * H_ROW) + i * 1024);
         }
     };
-    // token scales: thread tid -> token tid >> 2, sub-blocks 2 (tid & 3), + 1
-    const int tm = tid >> 2, ts = 2 * (tid & 3);
+    // token scales: thread tid -> row tid >> 2 of the stage (slot and token), sub-blocks 2 (tid & 3), + 1
+    const int tm = tid >> 2, ts = 2 * (tid & 3), tslot = SB > 1 ? tm / (32 * T) : 0, ttok = SB > 1 ? tm % (32 * T) : tm;
     const uint32_t* dtile = ads + m0 * nb;
-    const uint32_t doff = (uint32_t)(((m0 + tm < M) ? tm : M - 1 - m0) * nb + ts);
-    auto load_d = [&](int64_t kb) { return *reinterpret_cast<const v2u*>(dtile + kb * 8 + doff); };
+    const uint32_t doff = (uint32_t)(((m0 + ttok < M) ? ttok : M - 1 - m0) * nb + ts);
+    auto load_d = [&](int64_t kb) {
+        const uint32_t ob = SB > 1 ? 8u * (uint32_t)min<int64_t>(kb + tslot, bpr - 1) : 0u;
+        return *reinterpret_cast<const v2u*>(dtile + (SB > 1 ? 0 : kb * 8) + (doff + ob));
+    };
     // copy 1 (lane half 1, which meets the weight scale's low half) has 0
     // for a non-finite d_x, so that no Inf meets a zero low half (0 * Inf);
     // such a token's outputs are recomputed at the end (nonfinite_fixup), and
     // nf records that this thread saw one among the tile's own tokens
-    const bool own_token = tm < 32 * T && m0 + tm < M;
+    const bool own_token = ttok < 32 * T && m0 + ttok < M;
     bool nf = false;
     auto store_d = [&](v2u d, uint8_t* stage) {
         uint32_t* t = reinterpret_cast<uint32_t*>(stage + HStage<TOK>::t_off) + tm * 8 + ts;
@@ -436,7 +448,8 @@ __device__ __forceinline__ void f16_tile(const uint8_t* __restrict__ W, float* _
     HWeights w, wn;
     load_w(w, 0);
     if (bpr > 1) load_w(wn, 1);
-    issue_x(0, 0);
+#pragma unroll
+    for (int i = 0; i < SB; ++i) issue_x(i, 0, i);
     {
         const v2u d0 = load_d(0);
         __builtin_amdgcn_s_waitcnt(0);
@@ -444,43 +457,76 @@ __device__ __forceinline__ void f16_tile(const uint8_t* __restrict__ W, float* _
     }
     __syncthreads();
 
-    // one super-block from stage kb & 1 while super-block kb + 1 streams into
-    // the other; wc holds kb's weights, wo kb + 1's
-    // The loads are issued unconditionally (past the end they repeat the last
-    // super-block into registers and a stage that nothing reads any more), so
-    // that every iteration issues the same sequence: 2T copies + 1 token-scale
-    // load at the start, 5 weight loads after sub-block 2; the wait before the
-    // barrier then leaves exactly the 5 weight loads in flight.
-    auto superblock = [&](int64_t kb, HWeights& wc) {
-        const int cur = (int)(kb & 1);
-        const int64_t kb1 = min(kb + 1, bpr - 1), kb2 = min(kb + 2, bpr - 1);
-        issue_x(kb1, cur ^ 1);
-        v2u dnext = load_d(kb1);
-        f16_superblock<kDebug, T, TOK>(stages[cur], smem, wc, acc, kh, h, col, lane, kb, m0, M, n, N, nb, dbg,
-                               [&](HWeights& g) { load_w(g, kb2); });
-        // this thread's direct-to-LDS copies and token scales have landed; the
-        // 5 weight loads of super-block kb + 2, issued after them, may still
-        // be in flight (vmcnt counts completions in issue order)
+    // super-block kb (slot i of stage cur, weights wc) of the tile
+    auto superblock = [&](int64_t kb, int cur, int i, HWeights& wc) {
+        const int64_t kb2 = min(kb + 2, bpr - 1);
+        const uint8_t* st = stages[cur];
+        f16_superblock<kDebug, T, TOK>(st + i * (32 * T * H_ROW), st + HStage<TOK>::t_off + i * (32 * T * 32), smem, wc,
+                                       acc, kh, h, col, lane, kb, m0, M, n, N, nb, dbg,
+                                       [&](HWeights& g) { load_w(g, kb2); });
+    };
+    // the end of a stage: this thread's direct-to-LDS copies and token scales
+    // for the next one have landed; the 5 weight loads of super-block kb + 2,
+    // issued after them, may still be in flight (vmcnt counts completions in
+    // issue order)
+    auto end_stage = [&](v2u dnext, int cur, bool more) {
         __builtin_amdgcn_s_waitcnt(kVmcnt5);
         // keep the conversion of the token scales here: hoisted next to their
         // load it would need a vmcnt(0) there, i.e. wait for the whole next
         // stage before computing this one
         asm volatile("" : "+v"(dnext));
-        if (kb + 1 < bpr) store_d(dnext, stages[cur ^ 1]);
+        if (more) store_d(dnext, stages[cur ^ 1]);
         __syncthreads();
     };
-    // two super-blocks per iteration, so that the weight registers swap
-    // roles without copies (a copy of a register still being loaded would
-    // have to wait for the load)
-    // (an odd last super-block is peeled off, so that the loop is always
-    // entered from the second half: the compiler's own waits then know which
-    // weight loads are still in flight)
-    int64_t kb = 0;
-    for (; kb + 1 < bpr; kb += 2) {
-        superblock(kb, w);
-        superblock(kb + 1, wn);
+    if constexpr (SB > 1) {
+        // SB super-blocks from stage cur while the next SB stream into the
+        // other one, their copies issued with the first (and second) of them,
+        // ahead of that super-block's weight loads
+        int cur = 0;
+        for (int64_t kg = 0; kg < bpr; kg += SB, cur ^= 1) {
+            const bool more = kg + SB < bpr;
+            v2u dnext{};
+#pragma unroll
+            for (int i = 0; i < SB; ++i) {
+                if (i > 0 && kg + i >= bpr) break;
+                if (more && 2 * i < SB) {
+                    if (i == 0) dnext = load_d(kg + SB);
+                    issue_x(kg + SB + 2 * i, cur ^ 1, 2 * i);
+                    issue_x(kg + SB + 2 * i + 1, cur ^ 1, 2 * i + 1);
+                }
+                superblock(kg + i, cur, i, i & 1 ? wn : w);
+            }
+            end_stage(dnext, cur, more);
+        }
+    } else {
+        // one super-block from stage kb & 1 while super-block kb + 1 streams
+        // into the other; wc holds kb's weights, the other set kb + 1's.  The
+        // loads are issued unconditionally (past the end they repeat the last
+        // super-block into registers and a stage that nothing reads any more),
+        // so that every iteration issues the same sequence: 2T copies + 1
+        // token-scale load at the start, 5 weight loads after sub-block 2; the
+        // wait before the barrier then leaves exactly the 5 weight loads in
+        // flight.
+        auto one = [&](int64_t kb, HWeights& wc) {
+            const int cur = (int)(kb & 1);
+            issue_x(kb + 1, cur ^ 1, 0);
+            const v2u dnext = load_d(min(kb + 1, bpr - 1));
+            superblock(kb, cur, 0, wc);
+            end_stage(dnext, cur, kb + 1 < bpr);
+        };
+        // two super-blocks per iteration, so that the weight registers swap
+        // roles without copies (a copy of a register still being loaded would
+        // have to wait for the load)
+        // (an odd last super-block is peeled off, so that the loop is always
+        // entered from the second half: the compiler's own waits then know which
+        // weight loads are still in flight)
+        int64_t kb = 0;
+        for (; kb + 1 < bpr; kb += 2) {
+            one(kb, w);
+            one(kb + 1, wn);
+        }
+        if (kb < bpr) one(kb, w);
     }
-    if (kb < bpr) superblock(kb, w);
 
     // the two sub-block halves of each row group add their partial sums:
     // kh = 0 finalises token blocks j < (T + 1) / 2, kh = 1 the others, each
