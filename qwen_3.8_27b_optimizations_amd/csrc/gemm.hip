@@ -793,19 +793,23 @@ static bool f16_fits(int64_t K) {
     return (int64_t)H_BN * (K / QK_K) * BLOCK_BYTES < (1ll << 32) && (int64_t)H_BM * 2 * K < (1ll << 32);
 }
 
-// Token counts of the GEMM entry that the small-batch kernel takes: all of its
-// range, where the GEMM's 128-row tiles leave much of the chip idle or unfed
+// Calls of the GEMM entry that the small-batch kernel takes: all of its range,
+// where the GEMM's 128-row tiles leave much of the chip idle or unfed
 // (us, GEMM against small-batch: gate + up M = 16 69 / 37, M = 32 77 / 47, M =
 // 64 77 / 70; 17408 -> 5120 79 / 22, 79 / 29, 79 / 44; 8192 -> 5120 M = 33
-// 41 / 20; q/k/v M = 64 34 / 33; the one loss is a single 17408-row matrix from
-// M = 57 on, 43 / 45.5, whose pair gains as much).
-static bool use_gemv_mfma_above_gemv(int64_t M) { return M > GEMV_MAX_COLS && M <= GM_MAX_COLS; }
+// 41 / 20; q/k/v M = 64 34 / 33) -- but not from M = 57 on above 16384 rows,
+// whose 512 row blocks fill the two workgroups that a CU holds there: the rest
+// would take a second round (N = 17408, M = 64 43.6 / 45.5, N = 24000, K = 2048
+// 22.6 / 25.0; N = 16384 35.0 / 31.5).
+static bool use_gemv_mfma_above_gemv(int64_t N, int64_t M) {
+    return M > GEMV_MAX_COLS && M <= (N > 16384 ? 56 : GM_MAX_COLS);
+}
 
 hipError_t launch_gemm(const uint8_t* W, const int8_t* aqs, const uint32_t* ads, const uint32_t* ahq, float* Y,
                        int64_t K, int64_t N, int64_t M, int64_t ldy_m, int64_t ldy_n, int32_t* dbg,
                        hipStream_t stream) {
     clear_launch_error();
-    if (use_gemv_mfma_above_gemv(M)) {
+    if (use_gemv_mfma_above_gemv(N, M)) {
         const hipError_t e = launch_gemv_mfma(W, aqs, ads, Y, K, N, M, ldy_m, ldy_n, dbg, stream);
         if (e != hipErrorNotSupported) return e;
     }
@@ -831,7 +835,17 @@ hipError_t launch_gemm_group(int count, const uint8_t* const* W, float* const* Y
     clear_launch_error();
     if (count < 1 || count > GEMV_GROUP_MAX) return hipErrorInvalidValue;
     const int64_t ldy_n = layout_mk ? 1 : M;
-    if (use_gemv_mfma_above_gemv(M)) {
+    int small = 0;  // matrices that go to the small-batch kernel
+    for (int i = 0; i < count; ++i) small += use_gemv_mfma_above_gemv(N[i], M) ? 1 : 0;
+    if (small > 0 && small < count) {  // both kernels: each matrix by itself
+        for (int i = 0; i < count; ++i) {
+            const hipError_t e = launch_gemm(W[i], aqs, ads, ahq, Y[i], K, N[i], M, layout_mk ? N[i] : 1, ldy_n, nullptr,
+                                             stream);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    if (small == count) {
         int64_t ldy_m[GEMV_GROUP_MAX];
         for (int i = 0; i < count; ++i) ldy_m[i] = layout_mk ? N[i] : 1;
         const hipError_t e = launch_gemv_mfma_group(count, W, Y, N, ldy_m, aqs, ads, K, M, ldy_n, nullptr, stream);

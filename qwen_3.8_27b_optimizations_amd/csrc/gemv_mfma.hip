@@ -263,8 +263,11 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
 // Waves per workgroup of an N-row matrix.  They fix a row's fp32 summation
 // order, so they follow the matrix's own shape and M, never the launch.
 //   * From 384 row blocks on (gate/up, N = 17408) the blocks alone nearly fill
-//     the chip: 8 waves each, 4 past 32 tokens, where a workgroup of 8 leaves
-//     no room for a second one.
+//     the chip: 8 waves each.  Past 32 tokens, where a workgroup of 8 leaves
+//     no room for a second one, 4 waves as soon as there are more blocks than
+//     CUs (N = 11827, K = 3072, M = 61: 8 waves would need a second round, the
+//     case 25.9 us against the GEMM's 23.8; with 4 the launch takes 21.4, the
+//     GEMM's 22.9).
 //   * Below, K is split further so that every CU has loads in flight: 12
 //     waves, 8 past 48 tokens (all that the LDS holds), 16 up to 8 tokens from
 //     K = 8192 on (as fast, with shorter sums).
@@ -275,7 +278,7 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
 static int gm_waves(int64_t N, int64_t K, int G) {
     const int64_t bpr = K / QK_K;
     const int narrow = G == 1 && bpr < 32 ? 12 : gm_max_waves(G);
-    const int w = (N + 31) / 32 >= 384 ? (G <= 4 ? 8 : 4) : narrow;
+    const int w = (N + 31) / 32 >= (G <= 4 ? 384 : 257) ? (G <= 4 ? 8 : 4) : narrow;
     return (int)std::max<int64_t>(4, std::min<int64_t>(w, bpr));
 }
 

@@ -12,11 +12,12 @@ pytestmark = pytest.mark.gpu
 
 # K, N, M: the first and last M of each 8-token step (two MFMAs per decode past 32); a row
 # block of 1, 20 and 32 rows and a ragged last one; one super-block, fewer than the waves, and a K whose
-# super-blocks do not divide among them; both sides of 384 row blocks
+# super-blocks do not divide among them; both sides of 384 and of 256 row blocks and of 16384 rows
 CASES = [(256, 1, 9), (256, 33, 16), (768, 70, 17), (2048, 95, 24), (2304, 64, 25), (5120, 129, 32),
          (8448, 40, 16), (768, 5120 + 7, 12), (512, 32 * 384, 10), (256, 32 * 383 - 5, 31), (512, 2048, 33),
          (768, 2049, 48), (256, 8191, 49), (1280, 2100, 64), (256, 32 * 384, 40), (768, 32 * 383 + 5, 41),
-         (3328, 90, 56), (5120, 33, 57), (512, 32 * 384 + 1, 64), (8192, 64, 8)]
+         (3328, 90, 56), (5120, 33, 57), (512, 32 * 384 + 1, 64), (8192, 64, 8),
+         (256, 8192, 50), (256, 8193, 34), (256, 16384, 64), (256, 16385, 56), (256, 16385, 57)]
 
 
 @pytest.mark.parametrize("K,N,M", CASES)
