@@ -18,8 +18,8 @@
 // matrix and all columns (8 G of them), and splits K over its waves: wave w takes the
 // super-blocks kb = w, w + waves, ... (at any moment the waves stream adjacent
 // super-blocks of the same rows), with no barrier before the final sum.  The
-// partial sums are added in wave order and the wave count follows the
-// matrix's own shape (gm_waves), so a row's bits depend neither on the rows
+// partial sums are added in a fixed order and the split follows the
+// matrix's own shape (gm_split), so a row's bits depend neither on the rows
 // per workgroup nor on what shares the launch.
 //   * Loads are coalesced (each of the 4 weight loads of a block covers the qs
 //     of 8 whole rows, the activation loads a token's 256 codes per 8 lanes)
@@ -41,10 +41,9 @@
 //     1/(2 pi) = 0x3E22F983, an inline constant in the middle of the binade
 //     [1/8, 1/4), so that sumi (|sumi| < 2^20) counts units of 2^-26 there and
 //     one exact subtraction leaves sumi * 2^-26; the weight scale carries 2^26.
-#include <algorithm>
-
 #include "iq4xs_device.h"
 #include "iq4xs_internal.h"
+#include "small_batch_plan.h"
 
 namespace iq4xs {
 
@@ -63,11 +62,11 @@ constexpr int gm_wave_lds(int G) { return 32 * GM_WROW + G * (8 * gm_arow(G) + 8
 
 constexpr int GM_ZERO_BITS = 0x3E22F983;  // the accumulator's zero (1/(2 pi) as a float)
 
-// Most waves of a workgroup (gm_waves).
-constexpr int gm_max_waves(int G) { return G == 1 ? 16 : G <= 6 ? 12 : 8; }
 // Waves per SIMD that the registers are held to (96 to 128 VGPRs up to G = 4,
-// 161 and 168 at 5 and 6, 226 and 246 at 7 and 8, where the LDS allows no more).
-constexpr int gm_waves_per_simd(int G, bool debug) { return G == 1 ? 5 : (G == 2 ? 4 : (debug || G > 6 ? 2 : G <= 4 ? 4 : 3)); }
+// 161 and 168 at 5 and 6, 226 and 246 at 7 and 8, where the LDS allows no more);
+// `more`: the debug export, or two sums per wave (116 VGPRs; two workgroups
+// of 8 waves a CU either way).
+constexpr int gm_waves_per_simd(int G, bool more) { return G == 1 ? (more ? 4 : 5) : (G == 2 ? 4 : (more || G > 6 ? 2 : G <= 4 ? 4 : 3)); }
 
 // The matrices of one launch (same K and activations): workgroups
 // [tile_end[i-1], tile_end[i]) run matrix i.  Entries past the group's count
@@ -81,8 +80,9 @@ struct GmGroup {
     int tile_end[GEMV_GROUP_MAX];
 };
 
-template <int G, bool kDebug>
-__global__ __launch_bounds__(64 * gm_max_waves(G)) __attribute__((amdgpu_waves_per_eu(gm_waves_per_simd(G, kDebug))))
+// kTwo: two partial sums per wave (GmSplit)
+template <int G, bool kDebug, bool kTwo>
+__global__ __launch_bounds__(64 * gm_max_waves(G)) __attribute__((amdgpu_waves_per_eu(gm_waves_per_simd(G, kDebug || kTwo))))
 void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const uint32_t* __restrict__ ads, int K,
                       int M, int rows, int64_t ldy_n, int32_t* __restrict__ dbg) {
     // sub-blocks unrolled together: above 16 tokens one at a time, since the
@@ -225,11 +225,21 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
             }
         }
     };
+    // with two sums the super-blocks go to acc and alt in turn
+    float alt[kTwo ? 4 * G : 1] = {};
     // every load is unconditional (past this wave's last super-block it repeats that one)
     if (wave < bpr) {
         load_x(wave, 0);
         load_w(wave);
         for (int kb = wave; kb < bpr; kb += waves) {
+            if constexpr (kTwo) {
+#pragma unroll
+                for (int e = 0; e < 4 * G; ++e) {
+                    const float other = alt[e];
+                    alt[e] = acc[e];
+                    acc[e] = other;
+                }
+            }
             const int kn = kb + waves < bpr ? kb + waves : kb;
             const v2u hd = wh;
             stage_x(0);
@@ -244,48 +254,48 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
             }
         }
     }
-    // the waves' partial sums, added in wave order
+    // the partial sums, added in wave order (with two per wave the even ones
+    // first), those of twelve waves in two chains of every other one
     __syncthreads();  // the staging is free
-    float* red = reinterpret_cast<float*>(gm_lds);  // [waves][4G][64]
+    float* red = reinterpret_cast<float*>(gm_lds);  // [waves, or 2 waves][4G][64]
     constexpr int PER = 4 * G * 64;
-    static_assert(PER * 4 <= gm_wave_lds(G), "the final sum fits the staging");
+    static_assert((kTwo ? 2 : 1) * PER * 4 <= gm_wave_lds(G), "the final sum fits the staging");
+    const int sums = kTwo ? 2 * waves : waves;
+    if constexpr (kTwo) {
+        const bool odd = ((bpr - wave + waves - 1) / waves & 1) == 0;  // the last super-block was an odd one
 #pragma unroll
-    for (int e = 0; e < 4 * G; ++e) red[wave * PER + e * 64 + lane] = acc[e];
+        for (int e = 0; e < 4 * G; ++e) {
+            red[wave * PER + e * 64 + lane] = odd ? alt[e] : acc[e];
+            red[(waves + wave) * PER + e * 64 + lane] = odd ? acc[e] : alt[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4 * G; ++e) red[wave * PER + e * 64 + lane] = acc[e];
+    }
     __syncthreads();
     for (int e = wave; e < 4 * G; e += waves) {  // uniform per wave
         float v = red[e * 64 + lane];
-        for (int w = 1; w < waves; ++w) v += red[w * PER + e * 64 + lane];
+        if (G == 1 && !kTwo && waves == 12) {
+            float u = red[PER + e * 64 + lane];
+#pragma unroll
+            for (int w = 2; w < 12; w += 2) {
+                v += red[w * PER + e * 64 + lane];
+                u += red[(w + 1) * PER + e * 64 + lane];
+            }
+            v += u;
+        } else {
+            for (int w = 1; w < sums; ++w) v += red[w * PER + e * 64 + lane];
+        }
         const int t = 8 * (e >> 2) + 4 * h + (e & 3);
         if (t < M && col < nrow) Y[(int64_t)t * ldy_m + (int64_t)(r0 + col) * ldy_n] = v;
     }
 }
 
-// Waves per workgroup of an N-row matrix.  They fix a row's fp32 summation
-// order, so they follow the matrix's own shape and M, never the launch.
-//   * From 384 row blocks on (gate/up, N = 17408) the blocks alone nearly fill
-//     the chip: 8 waves each.  Past 32 tokens, where a workgroup of 8 leaves
-//     no room for a second one, 4 waves as soon as there are more blocks than
-//     CUs (N = 11827, K = 3072, M = 61: 8 waves would need a second round, the
-//     case 25.9 us against the GEMM's 23.8; with 4 the launch takes 21.4, the
-//     GEMM's 22.9).
-//   * Below, K is split further so that every CU has loads in flight: 12
-//     waves, 8 past 48 tokens (all that the LDS holds), 16 up to 8 tokens from
-//     K = 8192 on (as fast, with shorter sums).
-// Measured, us per launch with 4 / 8 / 12 waves: gate + up M = 8 30.6 / 30.3 /
-// 33.4, M = 32 48.5 / 47.7 / 55.2, M = 33 55 / 75 / 70, M = 64 70 / 81; 17408
-// -> 5120 M = 8 32.5 / 21.0 / 18.7 (16 waves 19.1), M = 32 50 / 33 / 29, M = 33
-// 66 / 43 / 36, M = 64 59 / 44; q/k/v M = 64 30 / 33.
-static int gm_waves(int64_t N, int64_t K, int G) {
-    const int64_t bpr = K / QK_K;
-    const int narrow = G == 1 && bpr < 32 ? 12 : gm_max_waves(G);
-    const int w = (N + 31) / 32 >= (G <= 4 ? 384 : 257) ? (G <= 4 ? 8 : 4) : narrow;
-    return (int)std::max<int64_t>(4, std::min<int64_t>(w, bpr));
-}
-
 template <int G>
-static hipError_t launch_gm(const GmGroup& grp, dim3 grid, int waves, const int8_t* aqs, const uint32_t* ads,
+static hipError_t launch_gm(const GmGroup& grp, dim3 grid, GmSplit split, const int8_t* aqs, const uint32_t* ads,
                             int64_t K, int64_t M, int64_t rows, int64_t ldy_n, int32_t* dbg,
                             hipStream_t stream) {
+    const int waves = split.waves;
     const size_t lds = (size_t)waves * gm_wave_lds(G);
     static_assert(gm_max_waves(G) * gm_wave_lds(G) <= GM_LDS_MAX, "the staging fits a CU");
     auto launch = [&](auto kernel) -> hipError_t {
@@ -298,21 +308,17 @@ static hipError_t launch_gm(const GmGroup& grp, dim3 grid, int waves, const int8
                            ldy_n, dbg);
         return hipGetLastError();
     };
-    return dbg ? launch(&gemv_mfma_kernel<G, true>) : launch(&gemv_mfma_kernel<G, false>);
+    if constexpr (G == 1)
+        if (split.two) return dbg ? launch(&gemv_mfma_kernel<G, true, true>) : launch(&gemv_mfma_kernel<G, false, true>);
+    return dbg ? launch(&gemv_mfma_kernel<G, true, false>) : launch(&gemv_mfma_kernel<G, false, false>);
 }
 
-// The matrices of one wave count in one launch.
-static hipError_t launch_gm_waves(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
+// The matrices of one split in one launch.
+static hipError_t launch_gm_split(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
                                   const int64_t* ldy_m, const int8_t* aqs, const uint32_t* ads, int64_t K, int64_t M,
-                                  int64_t ldy_n, int32_t* dbg, int waves, hipStream_t stream) {
+                                  int64_t ldy_n, int32_t* dbg, GmSplit split, hipStream_t stream) {
     const int64_t cus = device_cu_count();
-    // Rows per workgroup: 32, fewer where that leaves CUs without one (N =
-    // 5120: 20 rows on 256 CUs against 160 blocks of 32); at least 8, since
-    // each workgroup decodes all 32 MFMA rows whatever it keeps (N = 1024, M =
-    // 8: 6.6 us with 8 rows against 7.0 with 4).
-    int64_t total = 0;
-    for (int i = 0; i < count; ++i) total += N[i];
-    const int64_t rows = std::max<int64_t>(8, std::min<int64_t>(32, (total + cus - 1) / cus));
+    const int64_t rows = gm_rows(count, N, cus);
     GmGroup grp{};
     int64_t wgs = 0;
     for (int i = 0; i < GEMV_GROUP_MAX; ++i) {
@@ -327,7 +333,7 @@ static hipError_t launch_gm_waves(int count, const uint8_t* const* W, float* con
     }
     const dim3 grid((unsigned)wgs);
 #define IQ4XS_GM(G) \
-    case G: return launch_gm<G>(grp, grid, waves, aqs, ads, K, M, rows, ldy_n, dbg, stream)
+    case G: return launch_gm<G>(grp, grid, split, aqs, ads, K, M, rows, ldy_n, dbg, stream)
     switch ((M + 7) / 8) {
         IQ4XS_GM(1);
         IQ4XS_GM(2);
@@ -353,18 +359,18 @@ hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* con
         return hipErrorNotSupported;
     for (int i = 0; i < count; ++i)
         if (N[i] < 1 || N[i] >= (1 << 30)) return hipErrorNotSupported;
-    // one launch per wave count
+    // one launch per split
     const int G = (int)((M + 7) / 8);
     bool done[GEMV_GROUP_MAX] = {};
     for (int i = 0; i < count; ++i) {
         if (done[i]) continue;
-        const int waves = gm_waves(N[i], K, G);
+        const GmSplit split = gm_split(N[i], K, G);
         const uint8_t* gW[GEMV_GROUP_MAX];
         float* gY[GEMV_GROUP_MAX];
         int64_t gN[GEMV_GROUP_MAX], gL[GEMV_GROUP_MAX];
         int n = 0;
         for (int j = i; j < count; ++j) {
-            if (done[j] || gm_waves(N[j], K, G) != waves) continue;
+            if (done[j] || !(gm_split(N[j], K, G) == split)) continue;
             gW[n] = W[j];
             gY[n] = Y[j];
             gN[n] = N[j];
@@ -372,7 +378,7 @@ hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* con
             ++n;
             done[j] = true;
         }
-        const hipError_t e = launch_gm_waves(n, gW, gY, gN, gL, aqs, ads, K, M, ldy_n, dbg, waves, stream);
+        const hipError_t e = launch_gm_split(n, gW, gY, gN, gL, aqs, ads, K, M, ldy_n, dbg, split, stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

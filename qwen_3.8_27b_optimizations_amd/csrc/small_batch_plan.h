@@ -1,0 +1,70 @@
+// small_batch_plan.h -- which calls the small-batch matrix-core kernel takes
+// and how it splits them.  Plain host arithmetic on the shape, in a header of
+// its own so that the host tests compile the same rules.
+#pragma once
+
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace iq4xs {
+
+// The choices that fix a row's summation order count row blocks against
+// MI355X's 256 CUs, so that a device or partition with another CU count gives
+// the same bits; grid shapes use the device's own count.
+constexpr int64_t GM_CHOICE_CUS = 256;
+
+// Most waves of a workgroup at G groups of 8 columns (gm_split).
+constexpr int gm_max_waves(int G) { return G == 1 ? 16 : G <= 6 ? 12 : 8; }
+
+// How K is split over the waves of a workgroup: `waves` waves, each with one
+// partial sum or (`two`) one for its even and one for its odd super-blocks.
+struct GmSplit {
+    int waves;
+    bool two;
+    bool operator==(const GmSplit& o) const { return waves == o.waves && two == o.two; }
+};
+
+// The split of an N-row matrix.  It fixes a row's fp32 summation order, so it
+// follows the matrix's own shape and M, never the launch.
+//   * From 384 row blocks on (gate/up, N = 17408) the blocks alone nearly fill
+//     the chip: 8 waves each.  Past 32 tokens, where a workgroup of 8 leaves
+//     no room for a second one, 4 waves as soon as there are more blocks than
+//     CUs (N = 11827, K = 3072, M = 61: 21.4 us against 25.9 with 8, which
+//     would need a second round).
+//   * Below, K is split further so that every CU has loads in flight: 12
+//     waves, 8 past 48 tokens, 16 up to 8 tokens from K = 8192 on (as fast,
+//     with shorter sums).
+// Measured, us per launch with 4 / 8 / 12 waves: gate + up M = 8 30.6 / 30.3 /
+// 33.4, M = 32 48.5 / 47.7 / 55.2, M = 33 55 / 75 / 70, M = 64 70 / 81; 17408
+// -> 5120 M = 8 32.5 / 21.0 / 18.7 (16 waves 19.1), M = 32 50 / 33 / 29, M = 33
+// 66 / 43 / 36, M = 64 59 / 44.
+//
+// Precision at M <= 8: sixteen partial sums below 512 row blocks have the
+// shorter chains (K = 17408: 1.33e-7 against 1.59e-7 with eight, rel. 2-norm
+// against 64 bits).  From 384 blocks on 8 waves keep them as two sums each,
+// added in the order of sixteen waves, with the bits and without the time of
+// those (12288 x 3328, M = 8: 9.2 us, 16 waves 11.2).  Twelve waves add their
+// sums in two chains (gemv_mfma.hip), which is as close as sixteen in one
+// (K = 3584: 0.83e-7 against 0.89e-7; one chain of twelve 0.93e-7).
+inline GmSplit gm_split(int64_t N, int64_t K, int G) {
+    const int64_t bpr = K / 256, blocks = (N + 31) / 32;
+    constexpr int64_t kLarge = 3 * GM_CHOICE_CUS / 2;  // 384 row blocks
+    int waves = G == 1 && bpr < 32 ? 12 : gm_max_waves(G);
+    if (G <= 4 && blocks >= kLarge) waves = 8;
+    if (G >= 5 && blocks > GM_CHOICE_CUS) waves = 4;
+    return {(int)std::max<int64_t>(4, std::min<int64_t>(waves, bpr)),
+            G == 1 && blocks >= kLarge && blocks < 2 * GM_CHOICE_CUS && bpr > 8};
+}
+
+// Rows per workgroup of a launch of `count` matrices: 32, fewer where that
+// leaves CUs without one (N = 5120: 20 rows on 256 CUs against 160 blocks of
+// 32); at least 8, since each workgroup decodes all 32 MFMA rows whatever it
+// keeps (N = 1024, M = 8: 6.6 us with 8 rows against 7.0 with 4).
+inline int64_t gm_rows(int count, const int64_t* N, int64_t cus) {
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) total += N[i];
+    return std::max<int64_t>(8, std::min<int64_t>(32, (total + cus - 1) / cus));
+}
+
+}  // namespace iq4xs

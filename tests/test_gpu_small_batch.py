@@ -41,3 +41,52 @@ def test_token_and_row_blocks(pkg, orc, K, N, M):
     assert m["rel_l2"] <= 1e-4 and not m["bad"], m
     assert torch.equal(Yd, Y) and torch.equal(Ykm.T, Y)
     assert torch.equal(Yg[0], Y) and torch.equal(Yg[1], Y2)
+
+
+def sums_in_sixteen(S, W, AQ, K, N, M):
+    """[M][N] fp32 outputs and their fp64 values from the exact sub-block sums, K's super-blocks dealt out to sixteen
+    partial sums that are added one after another: acc = fma(sumi, fl(d_w (ls - 32) d_x), acc) per sub-block."""
+    b, nsb = W.reshape(N, K // 256, 136), K // 32
+    d = b[:, :, :2].copy().view(np.float16)[..., 0].astype(np.float32)
+    hi = b[:, :, 2].astype(np.int32) | (b[:, :, 3].astype(np.int32) << 8)
+    ls = np.stack([((b[:, :, 4 + i // 2].astype(np.int32) >> (4 * (i % 2))) & 15) | (((hi >> (2 * i)) & 3) << 4)
+                   for i in range(8)], -1).reshape(N, nsb) - 32
+    sa = np.repeat(d, 8, 1) * ls.astype(np.float32)  # exact
+    dx = AQ.reshape(M, nsb, 36)[:, :, :2].copy().view(np.float16)[..., 0].astype(np.float32)
+    sumi = np.where(ls == 0, 0, S // np.where(ls == 0, 1, ls))  # exact: S is their product
+    term = sumi * (sa[None] * dx[:, None]).astype(np.float64)
+    parts = []
+    for w in range(16):
+        acc = np.zeros((M, N), np.float32)
+        for kb in range(w, K // 256, 16):
+            for s in range(8 * kb, 8 * kb + 8):
+                acc = (acc + term[:, :, s]).astype(np.float32)
+        parts.append(acc)
+    y = parts[0]
+    for p in parts[1:]:
+        y = y + p
+    return y, term.sum(-1)
+
+
+# K, N, M: 384 to 511 row blocks (eight waves of two sums each, an odd and an even number of
+# super-blocks, fewer than sixteen), and twelve waves at both ends of their range of K
+@pytest.mark.parametrize("K,N,M", [(17408, 12288, 8), (8192, 16352, 4), (2304, 12257, 7), (1280, 13000, 5),
+                                   (3328, 4096, 8), (3584, 2048, 6), (7936, 5120, 4)])
+def test_no_further_from_64_bits_than_sixteen_sums(pkg, orc, K, N, M):
+    dev = torch.device("cuda:0")
+    print(f"precision K={K} N={N} M={M}", flush=True)
+    W = pkg.synthetic_weights(K, N, seed=9000 + K, device=dev)
+    X = orc.gen_activations(K * M, seed=9100 + M, outliers=True).reshape(M, K)
+    AQ = orc.quantize_q8_1_batched(X, K, M, LAYOUT_MK)
+    ws = pkg.quantize_q8_1(torch.from_numpy(X).to(dev), K, M, LAYOUT_MK)
+    Y = pkg.mul_mat_q8_1(W, ws, K, N, M, LAYOUT_MK)
+    torch.cuda.synchronize()
+    R, row = 512, K // 256 * 136  # the last rows: those of a ragged block among them
+    Wr = W[(N - R) * row:].cpu().numpy()
+    want, exact = sums_in_sixteen(orc.subblock_sums(Wr, AQ, K, R, M), Wr, AQ, K, R, M)
+    got = Y[:, N - R:].cpu().numpy()
+    err = lambda y: np.linalg.norm(y - exact) / np.linalg.norm(exact)  # noqa: E731
+    print(f"  against 64 bits {err(got):.3e}, sixteen sums {err(want):.3e}", flush=True)
+    if (N + 31) // 32 >= 384:  # the same sums in the same order
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    assert err(got) <= err(want)
