@@ -57,14 +57,24 @@ inline GmSplit gm_split(int64_t N, int64_t K, int G) {
             G == 1 && blocks >= kLarge && blocks < 2 * GM_CHOICE_CUS && bpr > 8};
 }
 
-// Rows per workgroup of a launch of `count` matrices: 32, fewer where that
-// leaves CUs without one (N = 5120: 20 rows on 256 CUs against 160 blocks of
-// 32); at least 8, since each workgroup decodes all 32 MFMA rows whatever it
-// keeps (N = 1024, M = 8: 6.6 us with 8 rows against 7.0 with 4).
+// Rows per workgroup of a launch of `count` matrices on `cus` CUs: the fewest
+// that give every CU at most one workgroup (N = 5120: 20 rows on 256 CUs
+// against 160 blocks of 32), 32 where that many do not fit.  Each matrix has a
+// ragged last block of its own, so the total alone does not tell: q/k/v of
+// 4096 + 512 + 512 rows have 257 workgroups of 20, and the last one is a
+// second round (K = 5120, M = 64: 29.1 us, with 21 rows 16.7).  At least 8,
+// since each workgroup decodes all 32 MFMA rows whatever it keeps (N = 1024,
+// M = 8: 6.6 us with 8 rows against 7.0 with 4).
 inline int64_t gm_rows(int count, const int64_t* N, int64_t cus) {
     int64_t total = 0;
     for (int i = 0; i < count; ++i) total += N[i];
-    return std::max<int64_t>(8, std::min<int64_t>(32, (total + cus - 1) / cus));
+    int64_t rows = std::max<int64_t>(8, std::min<int64_t>(32, (total + cus - 1) / cus));
+    for (; rows < 32; ++rows) {
+        int64_t wgs = 0;
+        for (int i = 0; i < count; ++i) wgs += (N[i] + rows - 1) / rows;
+        if (wgs <= cus) break;
+    }
+    return rows;
 }
 
 }  // namespace iq4xs

@@ -1,0 +1,29 @@
+// The small-batch kernel's host rules, from the library's own header: each
+// line of standard input is a question, each line of output its answer.
+//   rows CUS N...   -> rows per workgroup, workgroups of the launch
+#include <iostream>
+#include <sstream>
+#include <string>
+#include <vector>
+
+#include "small_batch_plan.h"
+
+int main() {
+    std::string line, what;
+    while (std::getline(std::cin, line)) {
+        std::istringstream in(line);
+        in >> what;
+        std::vector<int64_t> v;
+        for (int64_t x; in >> x;) v.push_back(x);
+        if (what == "rows") {
+            const int count = (int)v.size() - 1;
+            const int64_t rows = iq4xs::gm_rows(count, v.data() + 1, v[0]);
+            int64_t wgs = 0;
+            for (int i = 1; i <= count; ++i) wgs += (v[i] + rows - 1) / rows;
+            std::cout << rows << " " << wgs << "\n";
+        } else {
+            return 1;
+        }
+    }
+    return 0;
+}
