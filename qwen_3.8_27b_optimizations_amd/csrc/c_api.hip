@@ -328,7 +328,7 @@ int iq4xs_mul_mat_q8_1_group(int count, const void* const* W, float* const* Y, c
     const Planar p = planar_view(ws, K, M);
     const uint8_t* Wb[GEMV_GROUP_MAX];
     for (int i = 0; i < count; ++i) Wb[i] = static_cast<const uint8_t*>(W[i]);
-    if (M > GEMV_MAX_COLS)  // one GEMM launch: small matrices fill the big ones' last round
+    if (M > GEMV_MAX_COLS)
         return launch_gemm_group(count, Wb, Y, N, p.qs, p.ds, p.hq, K, M, layout == LAYOUT_MK, as_stream(stream));
     return launch_gemv_group(count, Wb, Y, N, p.qs, p.ds, K, M, layout == LAYOUT_MK, as_stream(stream));
 }

@@ -826,37 +826,45 @@ hipError_t launch_gemm(const uint8_t* W, const int8_t* aqs, const uint32_t* ads,
                : launch_f16_kernel<false, false>(grp, gx, aqs, ahq, ads, K, M, ldy_n, dbg, stream);
 }
 
-// One launch for `count` matrices sharing K and the activations: the round
-// planner sees the summed row tiles, so the small matrices fill CUs that the
-// big ones' last round leaves idle.
+// `count` matrices sharing K and the activations: those of the small-batch
+// kernel share its launches, the others one GEMM launch, whose round planner
+// sees the summed row tiles, so the small matrices fill CUs that the big ones'
+// last round leaves idle.
 hipError_t launch_gemm_group(int count, const uint8_t* const* W, float* const* Y, const int64_t* N, const int8_t* aqs,
                              const uint32_t* ads, const uint32_t* ahq, int64_t K, int64_t M, bool layout_mk,
                              hipStream_t stream) {
     clear_launch_error();
     if (count < 1 || count > GEMV_GROUP_MAX) return hipErrorInvalidValue;
     const int64_t ldy_n = layout_mk ? 1 : M;
-    int small = 0;  // matrices that go to the small-batch kernel
-    for (int i = 0; i < count; ++i) small += use_gemv_mfma_above_gemv(N[i], M) ? 1 : 0;
-    if (small > 0 && small < count) {  // both kernels: each matrix by itself
-        for (int i = 0; i < count; ++i) {
-            const hipError_t e = launch_gemm(W[i], aqs, ads, ahq, Y[i], K, N[i], M, layout_mk ? N[i] : 1, ldy_n, nullptr,
-                                             stream);
-            if (e != hipSuccess) return e;
+    const uint8_t* sW[GEMV_GROUP_MAX];
+    float* sY[GEMV_GROUP_MAX];
+    int64_t sN[GEMV_GROUP_MAX], sL[GEMV_GROUP_MAX];
+    int rest[GEMV_GROUP_MAX], small = 0, n = 0;
+    for (int i = 0; i < count; ++i) {
+        if (!use_gemv_mfma_above_gemv(N[i], M)) {
+            rest[n++] = i;
+            continue;
         }
-        return hipSuccess;
+        sW[small] = W[i];
+        sY[small] = Y[i];
+        sN[small] = N[i];
+        sL[small++] = layout_mk ? N[i] : 1;
     }
-    if (small == count) {
-        int64_t ldy_m[GEMV_GROUP_MAX];
-        for (int i = 0; i < count; ++i) ldy_m[i] = layout_mk ? N[i] : 1;
-        const hipError_t e = launch_gemv_mfma_group(count, W, Y, N, ldy_m, aqs, ads, K, M, ldy_n, nullptr, stream);
-        if (e != hipErrorNotSupported) return e;
+    if (small > 0) {
+        const hipError_t e = launch_gemv_mfma_group(small, sW, sY, sN, sL, aqs, ads, K, M, ldy_n, nullptr, stream);
+        if (e == hipErrorNotSupported) {  // past that kernel's offsets: the GEMM for all
+            for (n = 0; n < count; ++n) rest[n] = n;
+        } else if (e != hipSuccess) {
+            return e;
+        }
     }
+    if (n == 0) return hipSuccess;
     if (!f16_fits(K)) return hipErrorInvalidConfiguration;
     GemmGroup grp{};
     int64_t tiles = 0;
     for (int i = 0; i < GEMV_GROUP_MAX; ++i) {
-        const int j = i < count ? i : count - 1;  // unused entries repeat the last matrix, past every tile
-        if (i < count) tiles += (N[j] + H_BN - 1) / H_BN;
+        const int j = rest[i < n ? i : n - 1];  // unused entries repeat the last matrix, past every tile
+        if (i < n) tiles += (N[j] + H_BN - 1) / H_BN;
         if (tiles > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
         grp.W[i] = W[j];
         grp.Y[i] = Y[j];
@@ -864,7 +872,7 @@ hipError_t launch_gemm_group(int count, const uint8_t* const* W, float* const* Y
         grp.ldy_m[i] = layout_mk ? N[j] : 1;
         grp.tile_end[i] = (int)tiles;
     }
-    return launch_f16_kernel<false, true>(grp, tiles, aqs, ahq, ads, K, M, layout_mk ? 1 : M, nullptr, stream);
+    return launch_f16_kernel<false, true>(grp, tiles, aqs, ahq, ads, K, M, ldy_n, nullptr, stream);
 }
 
 // One v_mfma_i32_32x32x32_i8 on a 32x32 A and B (k-contiguous rows), C row-major:

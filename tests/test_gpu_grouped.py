@@ -91,3 +91,28 @@ def test_group_rejects_bad_arguments(pkg, dev):
     assert L.iq4xs_mul_mat_q8_1_group(2, wp, yp, n0, ws.data_ptr(), K, M, LAYOUT_MK, s) == inv
     assert L.iq4xs_mul_mat_q8_1_group(1, wp, yp, N5, ws.data_ptr(), K + 32, M, LAYOUT_MK, s) == inv
     torch.cuda.synchronize()
+
+
+# K, Ns, M and the launches they take: both kernels in one group are one launch of each, wherever the
+# matrices stand
+@pytest.mark.parametrize("K,Ns,M,launches", [(5120, (1024, 17408, 512, 2048), 57, 2),
+                                             (5120, (17408, 1024, 17408), 64, 2),
+                                             (5120, (8192, 1024, 1024), 64, 1), (512, (17408, 300), 70, 1)])
+def test_group_of_both_kernels(pkg, dev, K, Ns, M, launches):
+    import ctypes
+
+    print(f"launches K={K} Ns={Ns} M={M}", flush=True)
+    Ws = [pkg.synthetic_weights(K, N, seed=700 + i, device=dev) for i, N in enumerate(Ns)]
+    X = pkg.synthetic_activations(K * M, seed=78, outliers=True, device=dev)
+    ws = pkg.quantize_q8_1(X, K, M, LAYOUT_MK)
+    outs = pkg.mul_mat_q8_1_group(Ws, ws, K, list(Ns), M, LAYOUT_MK)
+    refs = [pkg.mul_mat_q8_1(W, ws, K, N, M, LAYOUT_MK) for W, N in zip(Ws, Ns)]
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(outs, refs))
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        pkg.mul_mat_q8_1_group(Ws, ws, K, list(Ns), M, LAYOUT_MK, outs=outs)
+    nodes = ctypes.c_size_t(0)
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    assert nodes.value == launches
