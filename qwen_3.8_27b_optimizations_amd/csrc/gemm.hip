@@ -793,26 +793,12 @@ static bool f16_fits(int64_t K) {
     return (int64_t)H_BN * (K / QK_K) * BLOCK_BYTES < (1ll << 32) && (int64_t)H_BM * 2 * K < (1ll << 32);
 }
 
-// Calls of the GEMM entry that the small-batch kernel takes: all of its range,
-// where the GEMM's 128-row tiles leave much of the chip idle or unfed
-// (us, GEMM against small-batch: gate + up M = 16 69 / 37, M = 32 77 / 47, M =
-// 64 77 / 70; 17408 -> 5120 79 / 22, 79 / 29, 79 / 44; 8192 -> 5120 M = 33
-// 41 / 20; q/k/v M = 64 34 / 33) -- but not from M = 57 on above 16384 rows,
-// whose 512 row blocks fill the two workgroups that a CU holds there: the rest
-// would take a second round (N = 17408, M = 64 43.6 / 45.5, N = 24000, K = 2048
-// 22.6 / 25.0; N = 16384 35.0 / 31.5).
-static bool use_gemv_mfma_above_gemv(int64_t N, int64_t M) {
-    return M > GEMV_MAX_COLS && M <= (N > 16384 ? 56 : GM_MAX_COLS);
-}
-
 hipError_t launch_gemm(const uint8_t* W, const int8_t* aqs, const uint32_t* ads, const uint32_t* ahq, float* Y,
                        int64_t K, int64_t N, int64_t M, int64_t ldy_m, int64_t ldy_n, int32_t* dbg,
                        hipStream_t stream) {
     clear_launch_error();
-    if (use_gemv_mfma_above_gemv(N, M)) {
-        const hipError_t e = launch_gemv_mfma(W, aqs, ads, Y, K, N, M, ldy_m, ldy_n, dbg, stream);
-        if (e != hipErrorNotSupported) return e;
-    }
+    if (M > GEMV_MAX_COLS && use_small_batch(N, K, M))
+        return launch_gemv_mfma(W, aqs, ads, Y, K, N, M, ldy_m, ldy_n, dbg, stream);
     if (!f16_fits(K)) return hipErrorInvalidConfiguration;
     GemmGroup grp{};
     grp.W[0] = W;
@@ -841,7 +827,7 @@ hipError_t launch_gemm_group(int count, const uint8_t* const* W, float* const* Y
     int64_t sN[GEMV_GROUP_MAX], sL[GEMV_GROUP_MAX];
     int rest[GEMV_GROUP_MAX], small = 0, n = 0;
     for (int i = 0; i < count; ++i) {
-        if (!use_gemv_mfma_above_gemv(N[i], M)) {
+        if (M <= GEMV_MAX_COLS || !use_small_batch(N[i], K, M)) {
             rest[n++] = i;
             continue;
         }
@@ -852,11 +838,7 @@ hipError_t launch_gemm_group(int count, const uint8_t* const* W, float* const* Y
     }
     if (small > 0) {
         const hipError_t e = launch_gemv_mfma_group(small, sW, sY, sN, sL, aqs, ads, K, M, ldy_n, nullptr, stream);
-        if (e == hipErrorNotSupported) {  // past that kernel's offsets: the GEMM for all
-            for (n = 0; n < count; ++n) rest[n] = n;
-        } else if (e != hipSuccess) {
-            return e;
-        }
+        if (e != hipSuccess) return e;
     }
     if (n == 0) return hipSuccess;
     if (!f16_fits(K)) return hipErrorInvalidConfiguration;

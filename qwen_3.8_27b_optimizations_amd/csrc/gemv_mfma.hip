@@ -43,7 +43,6 @@
 //     one exact subtraction leaves sumi * 2^-26; the weight scale carries 2^26.
 #include "iq4xs_device.h"
 #include "iq4xs_internal.h"
-#include "small_batch_plan.h"
 
 namespace iq4xs {
 

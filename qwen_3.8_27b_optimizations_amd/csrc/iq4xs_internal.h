@@ -2,6 +2,7 @@
 #pragma once
 
 #include "iq4xs_device.h"
+#include "small_batch_plan.h"
 
 namespace iq4xs {
 
@@ -41,7 +42,6 @@ hipError_t launch_gemv(const uint8_t* W, const int8_t* aqs, const uint32_t* ads,
 
 // Small-batch multiply on the int8 matrix cores (1 <= M <= GM_MAX_COLS, same
 // contract as launch_gemv); hipErrorNotSupported past its 32-bit offsets.
-constexpr int64_t GM_MAX_COLS = 64;
 hipError_t launch_gemv_mfma(const uint8_t* W, const int8_t* aqs, const uint32_t* ads, float* Y, int64_t K,
                             int64_t N, int64_t M, int64_t ldy_m, int64_t ldy_n, int32_t* dbg, hipStream_t stream);
 

@@ -14,6 +14,39 @@ namespace iq4xs {
 // the same bits; grid shapes use the device's own count.
 constexpr int64_t GM_CHOICE_CUS = 256;
 
+constexpr int64_t GM_MAX_COLS = 64;
+
+// Calls of the GEMM entry (M > 8) that the small-batch kernel takes: those
+// where neither the matrix alone, nor a pair of it (gate and up), nor it with
+// two eighths of its rows (q, k, v) is slower than on the GEMM.  The route
+// follows the matrix alone, since a grouped call has the bits of single ones;
+// up to 8192 rows it follows K and M alone, so that q, k and v go together.
+//   * The GEMM reads a weight once for all columns but needs about 256 tiles
+//     of 128 rows to fill the chip; this kernel fills it with 32-row blocks,
+//     and its time grows with the columns.  So it wins on few columns
+//     everywhere (us, GEMM / here: a pair of 17408 x 5120, M = 16 62 / 29), on
+//     many only where the GEMM's tiles are few (4096 x 17408, M = 64 79 / 46)
+//     or just past a round: pairs of 16384 to 24576 rows (17408 x 5120: M = 40
+//     71 / 51, M = 48 71 / 58), but not of 13312 (M = 40 40 / 47, M = 64 41 /
+//     52), and not a single matrix of 28672 (M = 40 41 / 47).
+//   * Short rows: with 5 to about 15 super-blocks most waves have one or two,
+//     and a second round of workgroups costs a full one (K = 1280: 28672 rows,
+//     M = 24 12.7 / 16.5, M = 32 13.0 / 20.1; a pair of 6144, M = 48 13.2 /
+//     17.3; K = 2304: a pair of 9216, M = 32 18.1 / 21.4, a pair of 8192, M =
+//     64 19.3 / 23.3), hence the least K, though a single matrix of 4096 rows
+//     is faster here below it too (K = 2304, M = 64 14.5 / 12.4).  Up to four
+//     super-blocks a workgroup has four waves, and more of them fit a CU.
+//   * The limits of the kernel's 32-bit offsets.
+inline bool use_small_batch(int64_t N, int64_t K, int64_t M) {
+    if (M > GM_MAX_COLS || N >= ((int64_t)1 << 30) || K >= ((int64_t)1 << 24)) return false;
+    constexpr int64_t kRound = 32 * GM_CHOICE_CUS;  // rows of one 32-row block per CU: 8192
+    if (M <= 24) return N <= 3 * kRound / 2 || K <= 1024 || K >= 1792;
+    if (M <= 32) return N <= kRound || K <= 1024 || K >= 5120;
+    if (M <= 40 && N <= kRound && (K <= 1024 || K >= 1792)) return true;
+    if (K < 4096) return false;
+    return N <= kRound || (M <= 48 && (N <= 3 * kRound / 2 || (N > 2 * kRound && N <= 3 * kRound)));
+}
+
 // Most waves of a workgroup at G groups of 8 columns (gm_split).
 constexpr int gm_max_waves(int G) { return G == 1 ? 16 : G <= 6 ? 12 : 8; }
 
@@ -30,15 +63,14 @@ struct GmSplit {
 //   * From 384 row blocks on (gate/up, N = 17408) the blocks alone nearly fill
 //     the chip: 8 waves each.  Past 32 tokens, where a workgroup of 8 leaves
 //     no room for a second one, 4 waves as soon as there are more blocks than
-//     CUs (N = 11827, K = 3072, M = 61: 21.4 us against 25.9 with 8, which
-//     would need a second round).
+//     CUs (up to 48 tokens: use_small_batch).
 //   * Below, K is split further so that every CU has loads in flight: 12
 //     waves, 8 past 48 tokens, 16 up to 8 tokens from K = 8192 on (as fast,
 //     with shorter sums).
 // Measured, us per launch with 4 / 8 / 12 waves: gate + up M = 8 30.6 / 30.3 /
-// 33.4, M = 32 48.5 / 47.7 / 55.2, M = 33 55 / 75 / 70, M = 64 70 / 81; 17408
-// -> 5120 M = 8 32.5 / 21.0 / 18.7 (16 waves 19.1), M = 32 50 / 33 / 29, M = 33
-// 66 / 43 / 36, M = 64 59 / 44.
+// 33.4, M = 32 48.5 / 47.7 / 55.2, M = 33 55 / 75 / 70; 17408 -> 5120 M = 8
+// 32.5 / 21.0 / 18.7 (16 waves 19.1), M = 32 50 / 33 / 29, M = 33 66 / 43 /
+// 36, M = 64 59 / 44.
 //
 // Precision at M <= 8: sixteen partial sums below 512 row blocks have the
 // shorter chains (K = 17408: 1.33e-7 against 1.59e-7 with eight, rel. 2-norm

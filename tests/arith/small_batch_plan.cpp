@@ -1,6 +1,7 @@
 // The small-batch kernel's host rules, from the library's own header: each
 // line of standard input is a question, each line of output its answer.
 //   rows CUS N...   -> rows per workgroup, workgroups of the launch
+//   small N K M     -> 1 if the GEMM entry's call goes to the small-batch kernel
 #include <iostream>
 #include <sstream>
 #include <string>
@@ -21,6 +22,8 @@ int main() {
             int64_t wgs = 0;
             for (int i = 1; i <= count; ++i) wgs += (v[i] + rows - 1) / rows;
             std::cout << rows << " " << wgs << "\n";
+        } else if (what == "small") {
+            std::cout << (iq4xs::use_small_batch(v[0], v[1], v[2]) ? 1 : 0) << "\n";
         } else {
             return 1;
         }

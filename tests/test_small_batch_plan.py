@@ -50,3 +50,32 @@ def test_one_round_of_workgroups_where_one_is_enough(ask, cus):
             assert wgs <= cus and (rows == 8 or at(rows - 1) > cus), (Ns, rows, wgs)
         else:
             assert rows == 32, (Ns, rows)
+
+
+# (N, K, M): the GEMM measured faster there, alone, in a pair or with two eighths of N beside it
+SLOWER = [(32768, 1280, 16), (13312, 1536, 20), (28672, 1280, 24), (9216, 2560, 32), (28672, 3072, 32),
+          (8192, 1280, 40), (13312, 5120, 40), (28672, 8192, 40), (2048, 768, 48), (8192, 1536, 48),
+          (10240, 3328, 48), (28672, 5120, 48), (8192, 2560, 62), (17408, 5120, 49), (17408, 1536, 56),
+          (11827, 1536, 57), (13824, 5120, 64), (151936, 4096, 56)]
+# and there this kernel, in all three
+FASTER = [(17408, 5120, 16), (5120, 17408, 16), (151936, 4096, 16), (151936, 1024, 24), (8192, 2560, 32),
+          (28672, 8192, 32), (5120, 8192, 33), (17408, 5120, 33), (12288, 4096, 40), (17408, 5120, 48),
+          (8192, 5120, 64), (1024, 5120, 64), (5120, 17408, 64)]
+
+
+def test_routes_by_measured_side(ask):
+    """Shapes on both sides of the lines; past the kernel's columns and 32-bit offsets the GEMM."""
+    cases = [(c, 0) for c in SLOWER] + [(c, 1) for c in FASTER]
+    cases += [((1024, 5120, 65), 0), ((1 << 30, 256, 16), 0), (((1 << 30) - 1, 256, 16), 1),
+              ((64, 1 << 24, 16), 0), ((64, (1 << 24) - 256, 16), 1)]
+    for (c, want), (got,) in zip(cases, ask([f"small {n} {k} {m}" for (n, k, m), _ in cases])):
+        assert got == want, c
+
+
+def test_q_k_and_v_take_one_route(ask):
+    """Up to 8192 rows the route does not depend on N: q, k and v of a grouped call stay in one launch."""
+    cases = [(k, m) for k in range(256, 17409, 256) for m in range(9, 66)]
+    rows = (8192, 4096, 1024, 1)
+    got = ask([f"small {n} {k} {m}" for k, m in cases for n in rows])
+    for i, c in enumerate(cases):
+        assert len({g[0] for g in got[len(rows) * i:len(rows) * (i + 1)]}) == 1, c
