@@ -358,7 +358,7 @@ __device__ __noinline__ void nonfinite_fixup(const uint8_t* __restrict__ W, floa
 // half-height tile of 4 waves, at most 64 tokens); wave w computes row group
 // w % RG on the sub-block half w / RG, so a row's arithmetic is the same in
 // both.
-template <bool kDebug, int T, int RG>
+template <bool kDebug, int T, int RG, int SB = 1>
 __device__ __forceinline__ void f16_tile(const uint8_t* __restrict__ W, float* __restrict__ Y, int64_t N,
                                          int64_t ldy_m, int tile0, const int8_t* __restrict__ aqs,
                                          const uint32_t* __restrict__ ahq,
@@ -367,12 +367,15 @@ __device__ __forceinline__ void f16_tile(const uint8_t* __restrict__ W, float* _
     static_assert(RG == 4 || (RG == 2 && T <= 2), "half-height tiles hold at most 64 tokens");
     constexpr int TOK = 32 * RG, STAGE = HStage<TOK>::bytes;
     constexpr int CPW = 8 * T / RG;  // 1 KB token copies per wave and super-block (16 T in all)
-    // Super-blocks per stage: a stage holds TOK rows of a token and a
-    // super-block, so a 128-row tile of 32 tokens takes four super-blocks
+    // SB super-blocks per stage: a stage holds TOK rows of a token and a
+    // super-block, so a 128-row tile of 32 tokens can take four super-blocks
     // between two barriers, with its copies further ahead (17408 -> 5120 at M =
     // 130: 98 -> 92 us).  Tiles of 64 tokens and half-height tiles measured
-    // 3-4 % slower with two.
-    constexpr int SB = T == 1 && RG == 4 ? 4 : 1;
+    // 3-4 % slower with two.  In the tail of a plan a tile of 32 tokens keeps
+    // one: four have to arrive there before it starts, at every CU at once and
+    // of tokens that few tiles share (5120 x 2048, M = 1024: 50.6 us with
+    // four, 47.7 with one).
+    static_assert(SB == 1 || (SB == 4 && T == 1 && RG == 4), "a stage holds TOK rows");
     uint8_t(*const stages)[STAGE] = reinterpret_cast<uint8_t(*)[STAGE]>(smem + H_LUT);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in an SGPR
@@ -641,7 +644,10 @@ __global__ __launch_bounds__(128 * RG) void gemm_f16_kernel(const GemmGroup grp,
         else f16_tile<kDebug, 2, 2>(W, Y, N, ldy_m, tile0, aqs, ahq, ads, K, M, ldy_n, bx, by, smem, dbg);
     } else {
         switch (sg.T) {
-            case 1: f16_tile<kDebug, 1, 4>(W, Y, N, ldy_m, tile0, aqs, ahq, ads, K, M, ldy_n, bx, by, smem, dbg); break;
+            case 1:
+                if (g == 0) f16_tile<kDebug, 1, 4, 4>(W, Y, N, ldy_m, tile0, aqs, ahq, ads, K, M, ldy_n, bx, by, smem, dbg);
+                else f16_tile<kDebug, 1, 4>(W, Y, N, ldy_m, tile0, aqs, ahq, ads, K, M, ldy_n, bx, by, smem, dbg);
+                break;
             case 2: f16_tile<kDebug, 2, 4>(W, Y, N, ldy_m, tile0, aqs, ahq, ads, K, M, ldy_n, bx, by, smem, dbg); break;
             case 3: f16_tile<kDebug, 3, 4>(W, Y, N, ldy_m, tile0, aqs, ahq, ads, K, M, ldy_n, bx, by, smem, dbg); break;
             default: f16_tile<kDebug, 4, 4>(W, Y, N, ldy_m, tile0, aqs, ahq, ads, K, M, ldy_n, bx, by, smem, dbg); break;
