@@ -21,15 +21,17 @@
 // nontemporal stores, which measured 59 us = 6.8 TB/s there (a device fill
 // reaches 6.9); smaller ones with plain stores, as fast up to 192 MiB (34.2
 // against 33.4 us) and left in the cache for their reader.
+#include "dequant_plan.h"
 #include "iq4xs_device.h"
 #include "iq4xs_internal.h"
 
 namespace iq4xs {
 
 template <bool kStream>
-__global__ __launch_bounds__(256) void dequant_iq4xs_kernel(const uint8_t* __restrict__ src, float* __restrict__ dst,
+__global__ __launch_bounds__(DEQUANT_WG) void dequant_iq4xs_kernel(const uint8_t* __restrict__ src, float* __restrict__ dst,
                                                             int64_t n_blocks) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    static_assert(DEQUANT_THREADS == 32, "t & 31 is the thread's part of its super-block");
     const int64_t b = t >> 5;
     if (b >= n_blocks) return;
     const int p = (int)(t & 31), g = p >> 3, c = p & 3, shift = p & 4;  // sub-block pair, qs dword, nibble
@@ -60,15 +62,22 @@ __global__ __launch_bounds__(256) void dequant_iq4xs_kernel(const uint8_t* __res
 
 hipError_t launch_dequant(const uint8_t* src, float* dst, int64_t n_blocks, hipStream_t stream) {
     clear_launch_error();
-    const int64_t threads = n_blocks * 32;
-    const int64_t grid = (threads + 255) / 256;
-    if (grid > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
     constexpr int64_t kCached = 192 * 1024;  // super-blocks of 1 KB of output: 192 MiB
-    if (n_blocks > kCached)
-        hipLaunchKernelGGL(dequant_iq4xs_kernel<true>, dim3((unsigned)grid), dim3(256), 0, stream, src, dst, n_blocks);
-    else
-        hipLaunchKernelGGL(dequant_iq4xs_kernel<false>, dim3((unsigned)grid), dim3(256), 0, stream, src, dst, n_blocks);
-    return hipGetLastError();
+    const bool stream_out = n_blocks > kCached;
+    for (int64_t done = 0; done < n_blocks;) {
+        const int64_t n = dequant_chunk(n_blocks - done);
+        const dim3 grid((unsigned)((n * DEQUANT_THREADS + DEQUANT_WG - 1) / DEQUANT_WG)), block(DEQUANT_WG);
+        const uint8_t* s = src + done * BLOCK_BYTES;
+        float* d = dst + done * QK_K;
+        if (stream_out)
+            hipLaunchKernelGGL(dequant_iq4xs_kernel<true>, grid, block, 0, stream, s, d, n);
+        else
+            hipLaunchKernelGGL(dequant_iq4xs_kernel<false>, grid, block, 0, stream, s, d, n);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        done += n;
+    }
+    return hipSuccess;
 }
 
 }  // namespace iq4xs

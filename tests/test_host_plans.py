@@ -1,5 +1,5 @@
-"""The host rules of the small-batch matrix-core kernel (csrc/small_batch_plan.h), compiled for the host and asked
-about many shapes."""
+"""The launchers' host rules (csrc/small_batch_plan.h, csrc/dequant_plan.h), compiled for the host and asked about
+many shapes."""
 import os
 import shutil
 import subprocess
@@ -14,9 +14,9 @@ CXX = os.environ.get("CXX", "g++")
 def ask(tmp_path_factory):
     if shutil.which(CXX) is None:
         pytest.skip("needs a host C++ compiler")
-    exe = str(tmp_path_factory.mktemp("plan") / "small_batch_plan")
+    exe = str(tmp_path_factory.mktemp("plan") / "host_plans")
     subprocess.run([CXX, "-std=c++17", "-O2", "-I" + os.path.join(ROOT, "qwen_3.8_27b_optimizations_amd", "csrc"),
-                    os.path.join(ROOT, "tests", "arith", "small_batch_plan.cpp"), "-o", exe], check=True)
+                    os.path.join(ROOT, "tests", "arith", "host_plans.cpp"), "-o", exe], check=True)
 
     def run(lines):
         r = subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True)
@@ -79,3 +79,14 @@ def test_q_k_and_v_take_one_route(ask):
     got = ask([f"small {n} {k} {m}" for k, m in cases for n in rows])
     for i, c in enumerate(cases):
         assert len({g[0] for g in got[len(rows) * i:len(rows) * (i + 1)]}) == 1, c
+
+
+def test_dequantiser_launches_hold_every_accepted_size(ask):
+    """Sizes whose threads pass the 2^32 that one launch must stay below (from 2^27 super-blocks, 128 GiB of output)
+    are divided; smaller ones stay one launch."""
+    sizes = [1, 8, 12345, 2 ** 27 - 9, 2 ** 27 - 8, 2 ** 27 - 7, 2 ** 27, 2 ** 27 + 1, 2 ** 28 - 1, 2 ** 31 - 1]
+    for n, got in zip(sizes, ask([f"dequant {n}" for n in sizes])):
+        blocks, threads = got[0::2], got[1::2]
+        assert sum(blocks) == n and max(threads) < 2 ** 32, n
+        assert all(b * 32 <= t for b, t in zip(blocks, threads)), n
+        assert len(blocks) == -(-n // (2 ** 27 - 8)), n
