@@ -29,13 +29,13 @@ GROUP_CASES = [  # K, Ns, M, layout
     (5120, (8192, 1024, 1024), 6, LAYOUT_KM),
     (5120, (17408, 17408), 8, LAYOUT_MK),         # gate/up: one matrix-core launch (8 waves each)
     (5120, (17408, 17408), 4, LAYOUT_KM),
-    (5120, (8192, 4096, 1024), 7, LAYOUT_MK),     # two matrix-core matrices (16 waves) share a launch
+    (5120, (8192, 4096, 1024), 7, LAYOUT_MK),     # two matrix-core matrices (12 waves) share a launch
     (5120, (8192, 1024, 1024), 8, LAYOUT_MK),     # at 8 columns the narrow k/v join q's launch
-    (5120, (17408, 8192, 2048, 512), 5, LAYOUT_KM),  # 8- and 16-wave launches, one tile launch
+    (5120, (17408, 8192, 2048, 512), 5, LAYOUT_KM),  # 8- and 12-wave launches, one tile launch
     (2048, (2048 + 7, 4096 + 31), 8, LAYOUT_MK),  # ragged last row blocks in a shared launch
     (8192, (5120,), 2, LAYOUT_KM),
     (1024, (40, 33, 9), 2, LAYOUT_MK),            # K < 2048: one launch per matrix
-    (2048, (300, 64), 20, LAYOUT_MK),             # M > 8: one GEMM launch
+    (2048, (300, 64), 20, LAYOUT_MK),             # small-batch kernel above 8 columns
     (5120, (8192, 1024, 1024), 512, LAYOUT_MK),   # q/k/v: the planner sees 80 row tiles, k alone 8
     (5120, (17408, 17408), 512, LAYOUT_KM),       # gate/up: a bulk of whole rounds and a tail segment
     (8192, (130, 4000, 64), 200, LAYOUT_MK),      # ragged tiles in every matrix

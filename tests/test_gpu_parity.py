@@ -328,8 +328,8 @@ def test_gemm_sums_and_outputs(pkg, orc, dev, K, N, M):
 EXTREME_D = np.array([0x0000, 0x0001, 0x0400, 0x3C00, 0x7BFF, 0x8400, 0x8001, 0xFBFF], np.uint16)
 
 
-# N, M: bs=1 tile GEMV, matrix-core GEMV (M = 4, 8), the GEMM on one and on many row tiles
-@pytest.mark.parametrize("N,M", [(2051, 1), (2051, 4), (2051, 8), (2051, 100), (128 * 145 + 3, 64)])
+# N, M: bs=1 tile GEMV, small-batch matrix-core kernel (4 to 40), the GEMM on few and on many row tiles
+@pytest.mark.parametrize("N,M", [(2051, 1), (2051, 4), (2051, 8), (2051, 20), (2051, 40), (2051, 100), (128 * 145 + 3, 64)])
 def test_extreme_weight_scales(pkg, orc, dev, N, M):
     """Each kernel family on weights whose fp16 d spans zero, subnormals and the largest
     finite values: the sub-block sums stay bit-exact and the outputs match the reference
@@ -549,8 +549,8 @@ def nonfinite_case(orc, M, inf_activation):
     return K, N, W, X
 
 
-# M: bs=1 tile GEMV, matrix-core GEMV (4, 8), fp16 matrix-core GEMM (64 one tile, 200 two token tiles)
-@pytest.mark.parametrize("M", [1, 4, 8, 64, 200])
+# M: bs=1 tile GEMV, small-batch matrix-core kernel (4 to 33), fp16 matrix-core GEMM in half-height tiles (64, 200)
+@pytest.mark.parametrize("M", [1, 4, 8, 16, 33, 64, 200])
 def test_nonfinite_weight_scales_keep_reference_classes(pkg, orc, dev, M):
     K, N, W, X = nonfinite_case(orc, M, inf_activation=False)
     AQ = orc.quantize_q8_1_batched(X, K, M, LAYOUT_MK)
@@ -561,9 +561,9 @@ def test_nonfinite_weight_scales_keep_reference_classes(pkg, orc, dev, M):
     check_classes(y_ref, Y.cpu().numpy().reshape(M, N), f"non-finite weight scales, M={M}")
 
 
-# M: matrix-core GEMV (4, 8) and the GEMM (64: one token tile; 200: more than one), on
-# weights that also carry non-finite scales
-@pytest.mark.parametrize("M", [4, 8, 64, 200])
+# M: small-batch matrix-core kernel (4 to 33) and the GEMM in half-height tiles (64, 200; full tiles:
+# test_gpu_gemm_stages.py), on weights that also carry non-finite scales
+@pytest.mark.parametrize("M", [4, 8, 16, 33, 64, 200])
 def test_infinite_activation_scale_keeps_reference_classes(pkg, orc, dev, M):
     print(f"Inf d_x M={M}", flush=True)
     K, N, W, X = nonfinite_case(orc, M, inf_activation=True)

@@ -1,7 +1,8 @@
 """The small-batch matrix-core kernel at the edges of its token blocks, row
 blocks and K split: int32 sub-block sums bit for bit against the oracle, fp32
 outputs to the path's tolerance (rel-L2 1e-4), every layout, the debug export
-and a grouped call bit-identical to the plain one."""
+and a grouped call bit-identical to the plain one.  Which calls the kernel
+takes is csrc/small_batch_plan.h's use_small_batch (test_host_plans.py)."""
 import numpy as np
 import pytest
 
@@ -10,14 +11,13 @@ from oracle.oracle import LAYOUT_KM, LAYOUT_MK, compute_metrics
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
-# K, N, M: the first and last M of each 8-token step (two MFMAs per decode past 32); a row
+# K, N, M: the first and last M of each 8-token step that takes short rows (two MFMAs per decode past 32); a row
 # block of 1, 20 and 32 rows and a ragged last one; one super-block, fewer than the waves, and a K whose
-# super-blocks do not divide among them; both sides of 384 and of 256 row blocks and of 16384 rows
+# super-blocks do not divide among them; then both sides of the lines on which the route to the GEMM lies
 CASES = [(256, 1, 9), (256, 33, 16), (768, 70, 17), (2048, 95, 24), (2304, 64, 25), (5120, 129, 32),
          (8448, 40, 16), (768, 5120 + 7, 12), (512, 32 * 384, 10), (256, 32 * 383 - 5, 31), (512, 2048, 33),
-         (768, 2049, 48), (256, 8191, 49), (1280, 2100, 64), (256, 32 * 384, 40), (768, 32 * 383 + 5, 41),
-         (3328, 90, 56), (5120, 33, 57), (512, 32 * 384 + 1, 64), (8192, 64, 8),
-         (256, 8192, 50), (256, 8193, 34), (256, 16384, 64), (256, 16385, 56), (256, 16385, 57)]
+         (4096, 2049, 48), (4352, 1000, 49), (4096, 2100, 64), (3328, 90, 40), (5120, 33, 57), (8192, 1024, 8),
+         (3840, 300, 41), (4096, 300, 41), (1024, 300, 40), (1280, 300, 40), (1792, 300, 40), (5120, 300, 65)]
 
 
 @pytest.mark.parametrize("K,N,M", CASES)
@@ -41,6 +41,40 @@ def test_token_and_row_blocks(pkg, orc, K, N, M):
     assert m["rel_l2"] <= 1e-4 and not m["bad"], m
     assert torch.equal(Yd, Y) and torch.equal(Ykm.T, Y)
     assert torch.equal(Yg[0], Y) and torch.equal(Yg[1], Y2)
+
+
+# K, N, M where every wave has several super-blocks, their counts unequal: each 8-token step with the waves that
+# its narrow and its wide matrices get (12 or 8 and 8 or 4), so that the next block's staging and loads, the reuse
+# of the two half blocks past 16 tokens and the final sum's reuse of the staging are run in each
+SEVERAL = [(6656, 100, 15), (4352, 12300, 16), (7168, 90, 20), (4352, 12289, 24), (8192, 70, 29), (5376, 12300, 32),
+           (8192, 100, 33), (4352, 8200, 40), (4352, 16400, 36), (8448, 100, 41), (4352, 8225, 48), (4352, 100, 50),
+           (5120, 8191, 56), (8448, 100, 64), (4352, 8192, 57), (8448, 1030, 7)]
+
+
+@pytest.mark.parametrize("K,N,M", SEVERAL)
+def test_several_super_blocks_per_wave(pkg, orc, K, N, M):
+    """Sampled rows (first, last and some between) against the oracle; a group with a narrow matrix, whose wave
+    count is another one where N is wide, against single calls."""
+    dev = torch.device("cuda:0")
+    print(f"several super-blocks K={K} N={N} M={M}", flush=True)
+    W = pkg.synthetic_weights(K, N, seed=7100 + K + N, device=dev)
+    X = orc.gen_activations(K * M, seed=8100 + M, outliers=True).reshape(M, K)
+    AQ = orc.quantize_q8_1_batched(X, K, M, LAYOUT_MK)
+    ws = pkg.quantize_q8_1(torch.from_numpy(X).to(dev), K, M, LAYOUT_MK)
+    S, Yd = pkg.subblock_sums(W, ws, K, N, M, pkg.PATH_GEMM if M > 8 else pkg.PATH_GEMV)
+    Y = pkg.mul_mat_q8_1(W, ws, K, N, M, LAYOUT_MK)
+    row = K // 256 * 136
+    n2 = 60 if M > 8 else 1030  # below 1024 rows 8 columns take another kernel
+    Yg = pkg.mul_mat_q8_1_group([W, W[:n2 * row]], ws, K, [N, n2], M, LAYOUT_MK)
+    Y2 = pkg.mul_mat_q8_1(W[:n2 * row], ws, K, n2, M, LAYOUT_MK)
+    torch.cuda.synchronize()
+    assert torch.equal(Yd, Y) and torch.equal(Yg[0], Y) and torch.equal(Yg[1], Y2)
+    rows = sorted({*range(0, min(N, 33)), *range(N // 2, min(N, N // 2 + 20)), *range(max(0, N - 40), N)})
+    at = torch.tensor(rows, device=dev)
+    Wr = np.ascontiguousarray(W.view(N, row)[at].cpu().numpy().ravel())
+    assert np.array_equal(S[:, at].cpu().numpy(), orc.subblock_sums(Wr, AQ, K, len(rows), M))
+    m = compute_metrics(orc.gemm_semantics(Wr, AQ, K, len(rows), M).T, Y[:, at].cpu().numpy())
+    assert m["rel_l2"] <= 1e-4 and not m["bad"], m
 
 
 def sums_in_sixteen(S, W, AQ, K, N, M):
