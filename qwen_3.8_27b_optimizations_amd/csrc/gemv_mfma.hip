@@ -259,7 +259,6 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
     float* red = reinterpret_cast<float*>(gm_lds);  // [waves, or 2 waves][4G][64]
     constexpr int PER = 4 * G * 64;
     static_assert((kTwo ? 2 : 1) * PER * 4 <= gm_wave_lds(G), "the final sum fits the staging");
-    const int sums = kTwo ? 2 * waves : waves;
     if constexpr (kTwo) {
         const bool odd = ((bpr - wave + waves - 1) / waves & 1) == 0;  // the last super-block was an odd one
 #pragma unroll
@@ -282,8 +281,11 @@ void gemv_mfma_kernel(const GmGroup grp, const int8_t* __restrict__ aqs, const u
                 u += red[(w + 1) * PER + e * 64 + lane];
             }
             v += u;
+        } else if constexpr (kTwo) {  // 8 waves
+#pragma unroll
+            for (int w = 1; w < 16; ++w) v += red[w * PER + e * 64 + lane];
         } else {
-            for (int w = 1; w < sums; ++w) v += red[w * PER + e * 64 + lane];
+            for (int w = 1; w < waves; ++w) v += red[w * PER + e * 64 + lane];
         }
         const int t = 8 * (e >> 2) + 4 * h + (e & 3);
         if (t < M && col < nrow) Y[(int64_t)t * ldy_m + (int64_t)(r0 + col) * ldy_n] = v;

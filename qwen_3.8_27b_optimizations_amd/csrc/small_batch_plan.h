@@ -76,17 +76,21 @@ struct GmSplit {
 // shorter chains (K = 17408: 1.33e-7 against 1.59e-7 with eight, rel. 2-norm
 // against 64 bits).  From 384 blocks on 8 waves keep them as two sums each,
 // added in the order of sixteen waves, with the bits and without the time of
-// those (12288 x 3328, M = 8: 9.2 us, 16 waves 11.2).  Twelve waves add their
-// sums in two chains (gemv_mfma.hip), which is as close as sixteen in one
-// (K = 3584: 0.83e-7 against 0.89e-7; one chain of twelve 0.93e-7).
+// those (12288 x 3328, M = 8: 9.3 us, 16 waves 11.2) -- where sixteen are
+// closer: with 9 to 15 super-blocks eight have up to 1.05 times their error,
+// with 16 to 24 as much (0.99 to 1.00), with more 1.02 times and rising.
+// Twelve waves add their sums in two chains (gemv_mfma.hip), which is closer
+// than sixteen in one (K = 3584: 0.83e-7 against 0.89e-7; one chain of twelve
+// 0.93e-7).
 inline GmSplit gm_split(int64_t N, int64_t K, int G) {
     const int64_t bpr = K / 256, blocks = (N + 31) / 32;
     constexpr int64_t kLarge = 3 * GM_CHOICE_CUS / 2;  // 384 row blocks
     int waves = G == 1 && bpr < 32 ? 12 : gm_max_waves(G);
     if (G <= 4 && blocks >= kLarge) waves = 8;
     if (G >= 5 && blocks > GM_CHOICE_CUS) waves = 4;
+    const bool longer = (bpr > 8 && bpr < 16) || bpr > 24;  // eight sums against sixteen, see above
     return {(int)std::max<int64_t>(4, std::min<int64_t>(waves, bpr)),
-            G == 1 && blocks >= kLarge && blocks < 2 * GM_CHOICE_CUS && bpr > 8};
+            G == 1 && blocks >= kLarge && blocks < 2 * GM_CHOICE_CUS && longer};
 }
 
 // Rows per workgroup of a launch of `count` matrices on `cus` CUs: the fewest
