@@ -570,7 +570,7 @@ def main() -> int:
                          "frac": round(b_bytes / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
                          "us_per_layer": round(us / args.layers, 2)}
         # the same rotation with q,k,v and gate,up each one grouped launch
-        # (matrix-core matrices of one wave count share a launch)
+        # (matrix-core matrices of one split of K share a launch)
         # group_args reads N from the outputs' element count: M rows of N
         bgroups = [(group_args(layers[l][0:3], [y[0] for y in yb[0:3]]),
                     group_args(layers[l][4:6], [y[0] for y in yb[4:6]])) for l in range(args.layers)]

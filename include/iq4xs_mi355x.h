@@ -51,9 +51,10 @@ extern "C" {
 #define IQ4XS_LAYOUT_MK 1 /* X[m*K + k], Y[m*N + n]  (ggml src1 / dst)                    */
 
 /* Kernel selection for iq4xs_mul_mat_q8_1 / iq4xs_subblock_sums */
-#define IQ4XS_PATH_AUTO -1 /* streaming GEMV for M <= 8, matrix-core GEMM above */
+#define IQ4XS_PATH_AUTO -1 /* IQ4XS_PATH_GEMV for M <= 8, IQ4XS_PATH_GEMM above */
 #define IQ4XS_PATH_GEMV 0  /* streaming GEMV (M <= 8 only)                   */
-#define IQ4XS_PATH_GEMM 1  /* matrix-core GEMM (any M)                       */
+#define IQ4XS_PATH_GEMM 1  /* matrix-core GEMM (any M); for 8 < M <= 64 the
+                            * small-batch matrix-core kernel where it is faster */
 
 /* ===================== standalone API (kernels/matmul_iq4xs) ===================== */
 
@@ -133,7 +134,7 @@ int gemm_iq4xs_lut_gpu(const void* W, const void* LUT, const float* X, float* Y,
 
 /* Replaces gemm_iq4xs_stock_dp4a_gpu, real_stock_dp4a_comparator.hip:505-548:
  * Y[n*M + m] = sum_k W[n,k] X[k*M + m].  M <= 8 runs the streaming GEMV,
- * larger M the matrix-core GEMM. */
+ * larger M the matrix-core GEMM (IQ4XS_PATH_GEMM). */
 int gemm_iq4xs_stock_dp4a_gpu(const void* W, const float* X, float* Y, int64_t K, int64_t N, int64_t M,
                               void* stream);
 
@@ -243,7 +244,11 @@ int iq4xs_rms_norm_mul_mat_swiglu(const void* W_gate, const void* W_up, int64_t 
                                   float* S, void* stream);
 
 /* Y = W * dequant(ws) from an already quantised workspace; `layout` selects
- * the Y layout; `path` is one of IQ4XS_PATH_*. */
+ * the Y layout; `path` is one of IQ4XS_PATH_*.  The same call gives the same
+ * bits every time.  The order in which a row's fp32 terms are added depends on
+ * N, K and M: above 64 columns it is one order for every M, below that it
+ * changes with the kernel and its split (by steps of 8 columns), so a column's
+ * last bits can differ between batch sizes. */
 int iq4xs_mul_mat_q8_1(const void* W, const void* ws, float* Y, int64_t K, int64_t N, int64_t M, int layout,
                        int path, void* stream);
 
@@ -251,17 +256,20 @@ int iq4xs_mul_mat_q8_1(const void* W, const void* ws, float* Y, int64_t K, int64
  * quantised activations in ws: Y[i] = W[i] * dequant(ws), Y[i] laid out as
  * `layout` selects.  For M <= 8 one launch of the streaming GEMV covers
  * every matrix (q/k/v, gate/up of a decode step) and pays the per-launch
- * fixed cost once; the matrices that take the matrix-core GEMV (M >= 4 and
- * N >= 2048, or M == 8 and N >= 1024) share one launch of it per wave count
- * (the count follows N),
- * the others one launch of the streaming GEMV.  For M > 8 one GEMM launch, whose
- * small matrices fill the CUs that the big ones' last round of tiles leaves
- * idle (a short last round lying in the last matrix is a second launch of
- * the small-tile kernel).  Each output is bit-identical to
- * iq4xs_mul_mat_q8_1 (path AUTO) on its own matrix.  W, Y, N are host arrays
- * of count entries.  No
- * counterpart in the reference, which runs every projection as its own
- * mul_mat. */
+ * fixed cost once; the matrices that take the small-batch matrix-core kernel
+ * (M >= 4 and N >= 2048, or M == 8 and N >= 1024) share its launches, the
+ * others one launch of the streaming GEMV.  For M > 8 the matrices share one
+ * GEMM launch, whose small matrices fill the CUs that the big ones' last round
+ * of tiles leaves idle, and up to 64 columns those that the small-batch kernel
+ * takes (a rule on N, K and M) share its launches instead.  That kernel has
+ * one launch per way of splitting K, which follows N, K and M: q/k/v and
+ * gate/up are one.  A group with matrices of both kernels pays a launch for
+ * each, and the narrow ones do not fill the wide ones' idle CUs: with q above
+ * 8192 rows, k and v beside it cost up to 40 % more than in one GEMM launch
+ * (12288 + 1536 + 1536 rows, K = 6144, M = 64: 54 against 40 us).  Each output
+ * is bit-identical to iq4xs_mul_mat_q8_1 (path AUTO) on its own matrix.  W, Y,
+ * N are host arrays of count entries.  No counterpart in the reference, which
+ * runs every projection as its own mul_mat. */
 int iq4xs_mul_mat_q8_1_group(int count, const void* const* W, float* const* Y, const int64_t* N, const void* ws,
                              int64_t K, int64_t M, int layout, void* stream);
 

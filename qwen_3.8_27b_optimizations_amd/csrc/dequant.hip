@@ -13,14 +13,18 @@
 // c (+ 4) takes qs dword c of both, the low (high) nibbles, so one 16-byte
 // store of the 8 lanes is sub-block 2g in output order and the next 2g + 1;
 // 32 threads share a super-block and read its 8-byte header.  (One lane for
-// both nibbles wrote 16-byte pieces 32 bytes apart: 5.2 against 5.8 TB/s on
-// 5120 x 17408, 78 against 70 us.)  Codes are decoded with the GEMV's v_perm
-// tables (decode_codes_x), one nibble at a time.
+// both nibbles wrote 16-byte pieces 32 bytes apart: 5120 x 17408 in 75.0 us,
+// whole lines 68.7.)  Codes are decoded with the GEMV's v_perm tables
+// (decode_codes_x), one nibble at a time.
 //
 // An output too large to stay in the 256 MB Infinity Cache is written with
-// nontemporal stores, which measured 59 us = 6.8 TB/s there (a device fill
-// reaches 6.9); smaller ones with plain stores, as fast up to 192 MiB (34.2
-// against 33.4 us) and left in the cache for their reader.
+// nontemporal stores: 56.0 us for 5120 x 17408 (340 MiB of output, the 45 MiB
+// of weights in the cache between passes; a device fill of that size takes
+// 53.1), 42.5 against 51.7 plain for 256 MiB.  Smaller ones are written with
+// plain stores, which leave them in the cache for their reader and take as
+// long where one buffer is written again and again (192 MiB 33.2 us plain,
+// 32.8 nontemporal; 128 MiB 23.0, 23.3); over several buffers nontemporal ones
+// would be faster on their own (192 MiB 39.7 plain, 32.4).
 #include "dequant_plan.h"
 #include "iq4xs_device.h"
 #include "iq4xs_internal.h"

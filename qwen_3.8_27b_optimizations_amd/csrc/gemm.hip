@@ -659,7 +659,10 @@ __global__ __launch_bounds__(128 * RG) void gemm_f16_kernel(const GemmGroup grp,
 // busy, for the round planner below (per-tile work is T token blocks against
 // the same weight decode, DMA and barrier cost per super-block).  Measured
 // on q_proj (K = 5120) at M = 512 with every workgroup of one size: 1, 2, 3
-// or 4 token blocks in 35.9, 47.4, 57.7, 77.3 us per round.
+// or 4 token blocks in 35.9, 47.4, 57.7, 77.3 us per round.  The first is the
+// tile of one super-block per stage, the one of a tail; a launch that begins
+// with one-block tiles runs them up to 10 % faster (four per stage), which no
+// plan counts on.
 static double f16_tile_cost(int T) {
     static const double c[5] = {0.0, 0.46, 0.61, 0.75, 1.0};
     return c[T < 1 ? 1 : (T > 4 ? 4 : T)];

@@ -62,7 +62,7 @@ constexpr int gm_wave_lds(int G) { return 32 * GM_WROW + G * (8 * gm_arow(G) + 8
 constexpr int GM_ZERO_BITS = 0x3E22F983;  // the accumulator's zero (1/(2 pi) as a float)
 
 // Waves per SIMD that the registers are held to (96 to 128 VGPRs up to G = 4,
-// 161 and 168 at 5 and 6, 226 and 246 at 7 and 8, where the LDS allows no more);
+// 161 and 168 at 5 and 6, 226 and 246 at 7 and 8);
 // `more`: the debug export, or two sums per wave (116 VGPRs; two workgroups
 // of 8 waves a CU either way).
 constexpr int gm_waves_per_simd(int G, bool more) { return G == 1 ? (more ? 4 : 5) : (G == 2 ? 4 : (more || G > 6 ? 2 : G <= 4 ? 4 : 3)); }

@@ -48,10 +48,10 @@ hipError_t launch_gemv_mfma(const uint8_t* W, const int8_t* aqs, const uint32_t*
 // Matrices run together by one grouped GEMV launch (same K, same activations).
 constexpr int GEMV_GROUP_MAX = 4;
 
-// The matrix-core GEMV over count <= GEMV_GROUP_MAX matrices, one launch per
-// wave count (which follows each matrix's own shape)
-// (Y[i] element (m, n) at Y[i][m*ldy_m[i] + n*ldy_n]).  dbg only with
-// count == 1.  Outputs are bit-identical to one launch per matrix.
+// The small-batch kernel over count <= GEMV_GROUP_MAX matrices, one launch per
+// split of K (gm_split, which follows each matrix's own shape); Y[i] element
+// (m, n) at Y[i][m*ldy_m[i] + n*ldy_n].  dbg only with count == 1.  Outputs
+// are bit-identical to one launch per matrix.
 hipError_t launch_gemv_mfma_group(int count, const uint8_t* const* W, float* const* Y, const int64_t* N,
                                   const int64_t* ldy_m, const int8_t* aqs, const uint32_t* ads, int64_t K,
                                   int64_t M, int64_t ldy_n, int32_t* dbg, hipStream_t stream);

@@ -65,8 +65,8 @@ struct GmSplit {
 //     no room for a second one, 4 waves as soon as there are more blocks than
 //     CUs (up to 48 tokens: use_small_batch).
 //   * Below, K is split further so that every CU has loads in flight: 12
-//     waves, 8 past 48 tokens, 16 up to 8 tokens from K = 8192 on (as fast,
-//     with shorter sums).
+//     waves, 8 past 48 tokens (226 and 246 registers leave two waves per
+//     SIMD), 16 up to 8 tokens from K = 8192 on (as fast, with shorter sums).
 // Measured, us per launch with 4 / 8 / 12 waves: gate + up M = 8 30.6 / 30.3 /
 // 33.4, M = 32 48.5 / 47.7 / 55.2, M = 33 55 / 75 / 70; 17408 -> 5120 M = 8
 // 32.5 / 21.0 / 18.7 (16 waves 19.1), M = 32 50 / 33 / 29, M = 33 66 / 43 /
