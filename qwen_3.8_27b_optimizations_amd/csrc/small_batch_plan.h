@@ -41,7 +41,7 @@ inline bool use_small_batch(int64_t N, int64_t K, int64_t M) {
     if (M > GM_MAX_COLS || N >= ((int64_t)1 << 30) || K >= ((int64_t)1 << 24)) return false;
     constexpr int64_t kRound = 32 * GM_CHOICE_CUS;  // rows of one 32-row block per CU: 8192
     if (M <= 24) return N <= 3 * kRound / 2 || K <= 1024 || K >= 1792;
-    if (M <= 32) return N <= kRound || K <= 1024 || K >= 5120;
+    if (M <= 32) return N <= kRound || K <= 1024 || K >= (N <= 3 * kRound / 2 ? 4608 : 5120);
     if (M <= 40 && N <= kRound && (K <= 1024 || K >= 1792)) return true;
     if (K < 4096) return false;
     return N <= kRound || (M <= 48 && (N <= 3 * kRound / 2 || (N > 2 * kRound && N <= 3 * kRound)));

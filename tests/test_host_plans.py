@@ -59,7 +59,7 @@ SLOWER = [(32768, 1280, 16), (13312, 1536, 20), (28672, 1280, 24), (9216, 2560, 
           (11827, 1536, 57), (13824, 5120, 64), (151936, 4096, 56)]
 # and there this kernel, in all three
 FASTER = [(17408, 5120, 16), (5120, 17408, 16), (151936, 4096, 16), (151936, 1024, 24), (8192, 2560, 32),
-          (28672, 8192, 32), (5120, 8192, 33), (17408, 5120, 33), (12288, 4096, 40), (17408, 5120, 48),
+          (12288, 4608, 32), (28672, 8192, 32), (5120, 8192, 33), (17408, 5120, 33), (12288, 4096, 40), (17408, 5120, 48),
           (8192, 5120, 64), (1024, 5120, 64), (5120, 17408, 64)]
 
 
